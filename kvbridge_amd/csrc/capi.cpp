@@ -192,10 +192,7 @@ hipError_t launch_split_fast(const SplitArgs& a, hipStream_t stream) {
 }
 
 const char* split_kernel_name(const SplitArgs& a, bool tiled, bool int8) {
-  if (!tiled) {
-    if (a.seq_starts) return int8 ? "split_generic_kernel<true, true>" : "split_generic_kernel<false, true>";
-    return int8 ? "split_generic_kernel<true, false>" : "split_generic_kernel<false, false>";
-  }
+  if (!tiled) return generic_kernel_name(a, int8);
   if (!force_f16() && i8_supported(a)) return i8_kernel_name(a);
   if (!force_f16() && i8_rows_supported(a)) return i8_rows_kernel_name(a);
   return lds_kernel_name(a);

@@ -1,125 +1,70 @@
-// Generic split-partial kernel: any valid Shape (dim 1..256, any page size,
-// any begin, int8 or fp32 KV, any GQA group).  It is the fallback behind
-// launch_attention for shapes the tiled MFMA kernel does not cover; the
-// arithmetic follows the per-split semantics of the reference
-// src/attention_shared.cu:42-209 / :213-293 (visible = k_pos <= q_pos, score =
-// (q . k_code) * k_scale * scale, weights exp(score - split max), numerator
-// weighted by v_scale), evaluated as an online softmax over 256-token chunks
-// so that one work-group can cover a split of any length.
+// Split partials of every valid shape that the tiled kernels do not take:
+// fp32 KV, other dims, misaligned buffers, and ragged batches over small
+// pages or with many head-rows.  The MFMA kernels (split_generic_mfma.h) serve
+// the shapes they can load in whole 16-byte pieces, the scalar kernel here
+// (split_generic.h) the rest: dims that are not a multiple of 4, pages that
+// are not a multiple of 16 tokens.
 //
-// Grid: x = row * q_heads + head, y = split, z = sequence of a batched call.
-// Block: 256 threads (4 waves).
+// Scalar kernel: grid x = row * q_heads + head, y = split, z = sequence of a
+// batched call; block of 256 threads (4 waves).
+#include <cstdio>
+
 #include "kernels.h"
 #include "batch.h"
-#include "device_common.h"
+#include "split_generic.h"
 
 namespace kvb {
+
+hipError_t launch_generic_i8(const SplitArgs& a, int nw, hipStream_t stream);
+hipError_t launch_generic_f32(const SplitArgs& a, int nw, hipStream_t stream);
+hipError_t preload_generic_i8();
+hipError_t preload_generic_f32();
+
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
-
-__device__ __forceinline__ float block_max(float x, float* red) {
-  x = wave_max(x);
-  const int wave = threadIdx.x >> 6;
-  __syncthreads();  // red is reused; previous readers must be done
-  if ((threadIdx.x & 63) == 0) red[wave] = x;
-  __syncthreads();
-  float r = red[0];
-#pragma unroll
-  for (int w = 1; w < kWaves; ++w) r = fmaxf(r, red[w]);
-  return r;
-}
-__device__ __forceinline__ float block_sum(float x, float* red) {
-  x = wave_sum(x);
-  const int wave = threadIdx.x >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[wave] = x;
-  __syncthreads();
-  float r = red[0];
-#pragma unroll
-  for (int w = 1; w < kWaves; ++w) r += red[w];
-  return r;
-}
-
-template <bool kInt8>
-__device__ __forceinline__ float kv_value(const void* base, uint32_t i) {
-  if constexpr (kInt8) return float(static_cast<const int8_t*>(base)[i]);
-  else return static_cast<const float*>(base)[i];
-}
 
 template <bool kInt8, bool VARLEN>
 __global__ __launch_bounds__(kThreads) void split_generic_kernel(SplitArgs a) {
   if constexpr (VARLEN) rebase_sequence(a, blockIdx.z);
-  __shared__ float q_s[256];
-  __shared__ float pw_s[kThreads];
-  __shared__ uint32_t vbase_s[kThreads];
-  __shared__ float red_s[2][kWaves];
+  __shared__ GenericLds<kThreads> lds;
+  split_generic_row<kInt8, kThreads>(a, blockIdx.x, blockIdx.y, lds);
+}
 
-  const uint32_t tid = threadIdx.x;
-  const uint32_t rh = blockIdx.x, split = blockIdx.y;
-  const uint32_t row = rh / a.q_heads, head = rh % a.q_heads;
-  const uint32_t kv = head / a.group;
-  const uint32_t D = a.dim, P = a.page_tokens;
+// Shapes of the MFMA kernels: K rows and V columns in dword-aligned 16-byte
+// loads (dim a multiple of 4, whole 16-token groups in a page), fp32 V slabs
+// within 32-bit byte offsets, and a grid of head-row blocks that fits grid.x.
+bool mfma_supported(const SplitArgs& a, bool int8) {
+  if (a.dim % 4 != 0 || a.page_tokens % 16 != 0) return false;
+  if (reinterpret_cast<uintptr_t>(a.k) % 4 != 0 || reinterpret_cast<uintptr_t>(a.v) % 4 != 0) return false;
+  if (!int8 && uint64_t(a.dim) * a.page_tokens >= (uint64_t(1) << 30)) return false;
+  const uint64_t blocks = (uint64_t(a.rows) * a.group + 15u) / 16u;
+  return a.kv_heads * blocks < (uint64_t(1) << 22);
+}
 
-  const uint64_t s0_64 = uint64_t(a.begin) + uint64_t(split) * a.split_tokens;
-  const uint32_t s0 = s0_64 < a.end ? uint32_t(s0_64) : a.end;
-  const uint32_t s1 = uint64_t(s0) + a.split_tokens < a.end ? s0 + a.split_tokens : a.end;
-  const int64_t qpos = a.q_positions[row];
-
-  if (tid < D) q_s[tid] = a.q[size_t(rh) * D + tid];
-  __syncthreads();
-
-  float m_run = neg_inf(), l_run = 0.f, acc = 0.f;
-  for (uint32_t c0 = s0; c0 < s1; c0 += kThreads) {
-    const uint32_t t = c0 + tid;
-    float score = neg_inf(), vsc = 0.f;
-    uint32_t vb = 0;
-    if (t < s1 && a.k_positions[t] <= qpos) {
-      uint32_t page = a.page_table[t / P];
-      page = page < a.pages ? page : a.pages - 1;
-      const uint32_t slot = t % P;
-      const uint32_t si = (page * a.kv_heads + kv) * P + slot;
-      float dot = 0.f;
-      for (uint32_t d = 0; d < D; ++d) dot = fmaf(q_s[d], kv_value<kInt8>(a.k, si * D + d), dot);
-      const float ks = kInt8 ? a.k_scales[si] : 1.f;
-      vsc = kInt8 ? a.v_scales[si] : 1.f;
-      score = dot * ks * a.scale;
-      vb = (page * a.kv_heads + kv) * D * P + slot;
-    }
-    const float cmax = block_max(score, red_s[0]);
-    const float m_new = fmaxf(m_run, cmax);
-    const float m_use = m_new == neg_inf() ? 0.f : m_new;
-    const float alpha = exp_e(m_run - m_use);  // m_run = -inf -> 0
-    const float w = exp_e(score - m_use);       // score = -inf -> 0
-    const float csum = block_sum(w, red_s[1]);
-    l_run = l_run * alpha + csum;
-    m_run = m_new;
-    pw_s[tid] = w * vsc;
-    vbase_s[tid] = vb;
-    __syncthreads();
-    if (tid < D) {
-      float part = 0.f;
-      const uint32_t cnt = s1 - c0 < uint32_t(kThreads) ? s1 - c0 : uint32_t(kThreads);
-      for (uint32_t j = 0; j < cnt; ++j) {
-        const float p = pw_s[j];
-        if (p != 0.f) part = fmaf(p, kv_value<kInt8>(a.v, vbase_s[j] + tid * P), part);
-      }
-      acc = fmaf(acc, alpha, part);
-    }
-    __syncthreads();
-  }
-  const size_t out = (size_t(rh) * a.splits + split) * (size_t(D) + 2);
-  if (tid == 0) {
-    a.scratch[out] = m_run;
-    a.scratch[out + 1] = l_run;
-  }
-  if (tid < D) a.scratch[out + 2 + tid] = acc;
+// Waves per work-group.  Up to two work-groups per CU: as many as the split
+// has tiles for, because a lone work-group is bound by latency (8,000 tokens,
+// dim 96, 128 work-groups of 8 tiles: split kernel 11.5 us with 8 waves,
+// 15.0 with 2).  Larger grids: two waves, so that four work-groups share a CU
+// and hide each other's prologue and combine (32 sequences of 100 .. 4,000
+// tokens, dim 128, 2,048 work-groups: 49 us per call with 2 waves, 51 with 4,
+// 73 with 8).  The state of dims above 128 takes a SIMD per wave.
+int mfma_waves(const SplitArgs& a, bool int8) {
+  const uint32_t tile = int8 ? 64u : 16u, tiles = (a.split_tokens - 1u) / tile + 1u;
+  const uint64_t blocks = (uint64_t(a.rows) * a.group + 15u) / 16u;
+  const uint64_t groups = blocks * a.kv_heads * a.splits * (a.seq_starts ? a.batch : 1u);
+  int nw = groups > 512u ? 2 : (a.dim <= 128 ? 8 : 4);
+  while (nw > 1 && uint32_t(nw) > tiles) nw /= 2;
+  return nw;
 }
 
 }  // namespace
 
 hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t stream) {
+  if (mfma_supported(a, int8)) {
+    const int nw = mfma_waves(a, int8);
+    return int8 ? launch_generic_i8(a, nw, stream) : launch_generic_f32(a, nw, stream);
+  }
   const bool varlen = a.seq_starts != nullptr;
   const dim3 grid(a.rows * a.q_heads, a.splits, varlen ? a.batch : 1u);
   if (int8 && varlen)
@@ -133,6 +78,18 @@ hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t strea
   return hipGetLastError();
 }
 
+// The family, and after a colon the MFMA instance that serves the call.
+const char* generic_kernel_name(const SplitArgs& a, bool int8) {
+  static thread_local char buf[128];
+  const char* const t = int8 ? "true" : "false";
+  const char* const v = a.seq_starts != nullptr ? "true" : "false";
+  const int at = std::snprintf(buf, sizeof(buf), "split_generic_kernel<%s, %s>", t, v);
+  if (mfma_supported(a, int8))
+    std::snprintf(buf + at, sizeof(buf) - at, ": split_generic_%s_kernel<%d, %d, %s>", int8 ? "i8" : "f32",
+                  a.dim <= 64 ? 64 : (a.dim <= 128 ? 128 : 256), mfma_waves(a, int8), v);
+  return buf;
+}
+
 hipError_t preload_generic() {
   const void* fns[] = {reinterpret_cast<const void*>(&split_generic_kernel<true, false>),
                        reinterpret_cast<const void*>(&split_generic_kernel<false, false>),
@@ -143,7 +100,8 @@ hipError_t preload_generic() {
     const hipError_t e = hipFuncGetAttributes(&attr, f);
     if (e != hipSuccess) return e;
   }
-  return hipSuccess;
+  const hipError_t e = preload_generic_i8();
+  return e != hipSuccess ? e : preload_generic_f32();
 }
 
 }  // namespace kvb

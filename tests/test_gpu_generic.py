@@ -1,0 +1,144 @@
+"""The generic family's MFMA kernels (fp32 KV, any dim that is a multiple of
+4, 16-token page groups) against the FP64 oracle, and against the scalar
+kernel on values a matrix product treats differently.
+
+Tolerance: the per-element gate |a - r| <= 3e-6 + 5e-5 |r| of fp32 arithmetic
+(examples/attention_bench.cu:127), as for the scalar kernel."""
+import zlib
+
+import numpy as np
+import pytest
+
+import kvbridge_amd as kvb
+from kvbridge_amd import workloads as W
+from oracle import oracle as O
+
+from helpers import DeviceCase, check_against_oracle, log
+from test_gpu_batched import DeviceBatch, check_sequence_vs_oracle
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # rows, q_heads, kv_heads, dim, page, tokens, begin, end, split, int8, query positions
+    (1, 4, 4, 4, 16, 200, 0, 200, 64, True, None),           # smallest dim; one wave per split
+    (1, 8, 2, 60, 16, 700, 3, 690, 128, True, None),         # padded 64-dim step, ragged range
+    (1, 8, 2, 68, 48, 1000, 17, 999, 256, True, None),       # just past a padded size, 48-token pages
+    (1, 17, 1, 72, 32, 900, 0, 900, 512, True, None),        # 17 head-rows: two blocks
+    (4, 16, 4, 112, 64, 1500, 0, 1500, 512, True, [100, 1400, -1, 777]),  # rows cut anywhere, one sees nothing
+    (1, 32, 8, 132, 16, 600, 0, 600, 256, True, None),       # four-wave instances
+    (1, 24, 4, 252, 16, 1100, 0, 1100, 1024, True, None),
+    (1, 8, 2, 96, 16, 20000, 0, 20000, 20000, True, None),   # one split of 313 tiles: several row windows
+    (1, 4, 4, 4, 16, 200, 0, 200, 64, False, None),
+    (1, 8, 2, 64, 16, 700, 5, 695, 128, False, None),
+    (1, 16, 1, 100, 48, 1000, 0, 1000, 256, False, None),
+    (4, 16, 4, 128, 32, 1500, 33, 1500, 512, False, [100, 1400, -1, 777]),
+    (1, 24, 4, 256, 64, 1100, 0, 1100, 512, False, None),
+    (2, 20, 2, 132, 16, 300, 0, 300, 512, False, None),      # 20 head-rows
+    (1, 8, 2, 64, 16, 9000, 0, 9000, 9000, False, None),     # one split of 563 tiles
+]
+
+
+@pytest.mark.parametrize("cfg", SHAPES)
+def test_generic_mfma_shapes(gpu, cfg):
+    rows, qh, kvh, d, p, t, b, e, st, int8, qpos = cfg
+    seed = zlib.crc32(repr(cfg).encode()) & 0xFFFF
+    case = W.synth_case(rows, qh, kvh, d, p, t, seed=seed, begin=b, end=e, int8=int8,
+                        qpos=None if qpos is None else np.array(qpos, np.int64))
+    dc = DeviceCase(case)
+    name = kvb.selected_kernel_name(case.shape, dc.inp, st)
+    log(f"generic mfma shape={case.shape.as_tuple()} split_tokens={st} kernel={name}")
+    assert ("split_generic_i8_kernel" if int8 else "split_generic_f32_kernel") in name
+    ref = O.fp64(case, threads=8)
+    mln, _, _ = dc.run_decode(st)
+    check_against_oracle(case, mln, "decode", ref, strict=True)
+    again, _, _ = dc.run_decode(st)
+    for x, y in zip(mln, again):  # bitwise repeatable
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+
+
+BATCHES = [
+    # rows, q_heads, kv_heads, dim, page, lengths, split, int8
+    (1, 32, 8, 128, 48, [300, 0, 1, 1000, 64], 256, True),
+    (4, 32, 8, 128, 64, [500, 129, 2], 256, True),      # 16 head-rows
+    (3, 24, 4, 256, 32, [200, 777], 128, True),         # 18 head-rows
+    (1, 8, 2, 80, 16, [100, 4000, 33] * 20, 64, True),  # many work-groups
+    (1, 8, 2, 64, 16, [300, 0, 17, 1000], 128, False),
+]
+
+
+@pytest.mark.parametrize("cfg", BATCHES)
+def test_generic_mfma_batches(gpu, cfg):
+    rows, qh, kvh, d, p, lengths, st, int8 = cfg
+    seed = zlib.crc32(repr(cfg).encode()) & 0xFFFF
+    bc = W.synth_batch(rows, qh, kvh, d, p, lengths, seed=seed, split_tokens=st, int8=int8)
+    db = DeviceBatch(bc.shape, bc.to_device("cuda:0"))
+    log(f"generic batch shape={bc.shape.as_tuple()} kernel={kvb.batch_kernel_name(bc.shape, db.inp)}")
+    m, l, n, _ = db.run(fused=False)
+    for b, t in enumerate(bc.lengths):
+        g = check_sequence_vs_oracle(bc, b, m, l, n, f"seq {b} (T={t})")
+        assert g is None or g["strict_pass"], (b, g)
+
+
+def _repage(case, page):
+    """The same tokens in pages of `page` slots (identity page table)."""
+    s = case.shape
+    tok = np.arange(s.tokens)
+    pg, sl = case.table[tok // s.page_tokens].astype(np.int64), tok % s.page_tokens
+    pages = -(-s.tokens // page)
+
+    def lay(rows, fill):  # [tokens, kv, ...] -> [pages, kv, page, ...]
+        out = np.full((pages * page,) + rows.shape[1:], fill, rows.dtype)
+        out[:s.tokens] = rows
+        return np.ascontiguousarray(np.moveaxis(out.reshape((pages, page) + rows.shape[1:]), 1, 2))
+
+    k = lay(case.k[pg, :, sl], 0)
+    v = np.ascontiguousarray(np.swapaxes(lay(case.v[pg, :, :, sl], 0), 2, 3))
+    ks, vs = lay(case.ks[pg, :, sl], 1), lay(case.vs[pg, :, sl], 1)
+    shape = s.copy(page_tokens=page, pages=pages)
+    return W.Case(shape, case.q, case.qpos, case.kpos, np.arange(pages, dtype=np.uint32), k, v, ks, vs)
+
+
+NON_FINITE = ["v_inf_zero_weight", "v_nan_masked", "k_nan", "k_inf", "q_nan", "scale_nan", "scale_inf_masked"]
+
+
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("what", NON_FINITE)
+def test_non_finite_values_match_the_scalar_kernel(gpu, what, int8):
+    """Infinities and NaN in Q, the cache or the scales: the same places are
+    non-finite as in the scalar kernel (which the same tokens in pages of 8
+    slots reach), and everything else agrees to fp32 rounding."""
+    case = W.synth_case(1, 8, 2, 96, 16, 400, seed=5, permute=True, int8=int8, qpos=[370])
+    tok = {"v_nan_masked": 380, "scale_inf_masked": 390}.get(what, 123)
+    pg, sl = int(case.table[tok // 16]), tok % 16
+    if what.startswith("v_"):
+        if int8:
+            case.vs[pg, 0, sl] = np.inf if what == "v_inf_zero_weight" else np.nan
+        else:
+            case.v[pg, 0, 5, sl] = np.inf if what == "v_inf_zero_weight" else np.nan
+        if what == "v_inf_zero_weight":  # a score far below the maximum: the weight underflows to 0
+            if int8:
+                case.ks[pg, 0, sl] *= np.float32(1e6)
+            else:
+                case.k[pg, 0, sl] *= np.float32(1e6)
+    elif what == "k_nan" or what == "k_inf":
+        bad = np.float32(np.nan if what == "k_nan" else np.inf)
+        if int8:
+            case.ks[pg, 0, sl] = bad
+        else:
+            case.k[pg, 0, sl, 7] = bad
+    elif what == "q_nan":
+        case.q[2 * 96 + 11] = np.nan
+    elif what == "scale_nan":
+        case.vs[pg, 0, sl] = np.nan
+    else:
+        case.ks[pg, 0, sl], case.vs[pg, 0, sl] = np.inf, np.nan
+    other = _repage(case, 8)
+    a, b = DeviceCase(case), DeviceCase(other)
+    name_a = kvb.selected_kernel_name(case.shape, a.inp, 128)
+    assert "_kernel<128" in name_a and ":" not in kvb.selected_kernel_name(other.shape, b.inp, 128)
+    for x, y, nm in zip(a.run_decode(128)[0], b.run_decode(128)[0], "mln"):
+        assert np.array_equal(np.isnan(x), np.isnan(y)) and np.array_equal(np.isinf(x), np.isinf(y)), nm
+        fin = np.isfinite(y)
+        log(f"  {what} int8={int8} {nm}: {np.count_nonzero(~fin)} non-finite")
+        if fin.any():
+            np.testing.assert_allclose(x[fin], y[fin], rtol=5e-5, atol=3e-6 * max(1.0, np.abs(y[fin]).max()))
