@@ -29,7 +29,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_rows_kernel(
   __shared__ __attribute__((aligned(16))) float lds[L::kFloats];
   const size_t rh = blockIdx.x;
   const float* const base = scratch + rh * splits * (D + 2);
-  merge_rows<D, kRowsWaves, 1, false>(
+  merge_rows<D, kRowsWaves, 1>(
       1u, splits, [&](uint32_t) { return base; }, lds,
       [&](uint32_t, uint32_t q, float4 nv, float mv, float lv) {
         if (q == 0) {

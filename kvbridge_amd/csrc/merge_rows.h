@@ -16,9 +16,6 @@
 // wave per row-head (lane = split) and shared through LDS; L is a wave tree
 // per pass, added in pass order.  The result is deterministic: it depends
 // only on S, D and the thread layout.
-//
-// AGENT: partials written by other work-groups of the running kernel (any
-// XCD) -- every load uses the agent-scope coherent policy (sc1).
 #pragma once
 #include <cstdint>
 
@@ -42,19 +39,10 @@ struct MergeRowsLayout {
 
 namespace merge_detail {
 
-constexpr int kAuxPlain = 0;
-constexpr int kAuxAgent = 16;  // sc1: the cache policy of an agent-scope atomic load
-
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const float* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, int(bytes), 0x00020000);
-}
-
-template <bool AGENT>
-__device__ __forceinline__ float load1(const float* p) {
-  if constexpr (AGENT) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else return *p;
 }
 
 }  // namespace merge_detail
@@ -63,12 +51,11 @@ __device__ __forceinline__ float load1(const float* p) {
 // emit(r, q, N (float4: columns 4q..4q+3), M, L) is called once per quad
 // of every row-head, by the thread that owns it.  lds: kFloats floats,
 // 16-byte aligned.  Every thread of the work-group must call this.
-template <int D, int NW, int RM, bool AGENT, typename RowBase, typename Emit>
+template <int D, int NW, int RM, typename RowBase, typename Emit>
 __device__ __forceinline__ void merge_rows(uint32_t R, uint32_t S, RowBase row_base, float* lds, Emit emit) {
   using L = MergeRowsLayout<D, NW, RM>;
   using merge_detail::u32x4;
   constexpr uint32_t W = D + 2;
-  constexpr int aux = AGENT ? merge_detail::kAuxAgent : merge_detail::kAuxPlain;
   float* const fs = lds;                                                   // [RM][kPS]
   float* const ml = lds + RM * L::kPS;                                     // [RM][4]: M, L
   float4* const part = reinterpret_cast<float4*>(lds + RM * L::kPS + 4 * RM);  // [kG][kQT]
@@ -85,7 +72,7 @@ __device__ __forceinline__ void merge_rows(uint32_t R, uint32_t S, RowBase row_b
     for (uint32_t h = wave; h < R; h += NW) {
       const float* b = row_base(h);
       float mx = neg_inf();
-      for (uint32_t j = lane; j < S; j += 64u) mx = fmaxf(mx, merge_detail::load1<AGENT>(b + size_t(j) * W));
+      for (uint32_t j = lane; j < S; j += 64u) mx = fmaxf(mx, b[size_t(j) * W]);
       mx = wave_max(mx);
       if (lane == 0) ml[4 * h] = mx;
     }
@@ -100,15 +87,15 @@ __device__ __forceinline__ void merge_rows(uint32_t R, uint32_t S, RowBase row_b
 #pragma unroll
     for (uint32_t k = 0; k < L::kK; ++k) {
       const uint32_t j = j0 + g + L::kG * k;
-      v[k] = __builtin_amdgcn_raw_buffer_load_b128(rs, int(((j < jmax ? j : jmax) * W + 2u + 4u * q) * 4u), 0, aux);
+      v[k] = __builtin_amdgcn_raw_buffer_load_b128(rs, int(((j < jmax ? j : jmax) * W + 2u + 4u * q) * 4u), 0, 0);
     }
     for (uint32_t h = wave; h < R; h += NW) {
       const float* b = row_base(h);
       const uint32_t j = j0 + lane;
       const bool in = lane < L::kPS && j < S;
       const float* pj = b + size_t(in ? j : 0u) * W;
-      const float mj = merge_detail::load1<AGENT>(pj);
-      const float lj = merge_detail::load1<AGENT>(pj + 1);
+      const float mj = pj[0];
+      const float lj = pj[1];
       const float mx = passes > 1u ? ml[4 * h] : wave_max(in ? mj : neg_inf());
       const float f = in && lj > 0.f ? exp_e(mj - mx) : 0.f;
       const float lsum = wave_sum(f * lj);

@@ -16,7 +16,8 @@
 // small per-wave LDS exchange area), so no VALU work is spent on padding
 // columns.
 //
-// Two passes per chunk of up to 4 tiles: the K images of the chunk are
+// Two passes per chunk of up to 4 tiles (NB = 1: one tile, for waves that
+// hold one or two): the K images of the chunk are
 // streamed first (scores kept in registers, exact chunk maximum), then the V
 // images; the int32 numerators therefore never need an online rescale and
 // are folded into fp32 once per chunk.
@@ -36,9 +37,9 @@
 // Partial layout and semantics are those of every split kernel here:
 // scratch[((row*q_heads + head)*splits + split)*(dim+2) + col], col 0 = split
 // max score (natural log units), 1 = sum of exp(score - max), 2.. =
-// sum of exp(score - max) * v_scale * v_code -- except in the single launch
-// whose merge takes the short path, which packs the same values differently
-// in the same scratch (PackedPartials below).
+// sum of exp(score - max) * v_scale * v_code -- except in the single launch,
+// which packs the same values differently in the same scratch
+// (PackedPartials below).
 #pragma once
 #include <cstdint>
 
@@ -46,7 +47,6 @@
 #include "batch.h"
 #include "device_common.h"
 #include "lds_stream.h"
-#include "merge_rows.h"
 
 namespace kvb {
 namespace {
@@ -56,7 +56,6 @@ using lds::u32x4_t;
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kTileTokens = 64;
-constexpr int kChunk = 4;                    // tiles per two-pass chunk
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr int32_t kRsrcWord3 = 0x00020000;   // raw 32-bit buffer, gfx9 dword3
 
@@ -222,7 +221,7 @@ __device__ __forceinline__ float ld_agent(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The single launch's short merge (at most 32 splits, one output column per
+// The single launch's merge (at most 32 splits, one output column per
 // thread) reads a packed partial layout of its own instead of the
 // [row-head][split][m, l, n] rows above (same size, internal to the call):
 //   m: scratch[rh*splits + j]             (RS = rows * q_heads * splits)
@@ -247,187 +246,85 @@ struct PackedPartials {
   }
 };
 
-// Whether the single launch's merge takes the short path (and so the packed
-// layout): every work-group of the kernel evaluates the same condition.
-template <int D, int NW>
-__device__ __forceinline__ bool short_merge(uint32_t ns, uint32_t head_rows) {
-  return ns <= 32u && head_rows * uint32_t(D) <= 64u * NW;
-}
-
 // Merge of all splits of one kv head's head-rows, by the last work-group,
 // with the reference merge semantics (src/attention_shared.cu:295-335):
-// M = max_j m_j; L = sum_{l_j > 0} e^{m_j - M} l_j; N[d] likewise (N summed
-// in split order, L by a wave tree); an all-empty head-row gives M = -inf,
+// M = max_j m_j; L = sum_{l_j > 0} e^{m_j - M} l_j; N[d] likewise (N in four
+// interleaved sums, L by a wave tree); an all-empty head-row gives M = -inf,
 // L = 0, N = 0.  Optional normalized output out = L > 0 ? N / L : 0 (fp32 or
 // fp16).  Splits 0 .. ns-1 are merged; a.splits is the partial stride.
-// f_s: LDS [8][32] split factors (the merge_rows area when that runs),
-// ml_s: LDS [8][2] (M, L).
-template <int D, int NW, int HS>
+// i8_fusable admits at most 32 splits, one output per thread and one head-row
+// per wave: straight-line code that requests every operand at once -- the
+// wave's (m_j, l_j) and the thread's 32 numerators, split indices clamped
+// instead of branched on -- so the merge costs one memory round trip.  The 64
+// outputs of a wave lie in one head-row (64 divides D), so every wave turns
+// its own head-row's (m_j, l_j) into the factors e^{m_j - M} (lane j holds
+// split j), without a work-group barrier.  f_s: LDS [NW][32] split factors.
+template <int D, int NW>
 __device__ __forceinline__ void fused_merge(const SplitArgs& a, uint32_t kv, uint32_t head_rows, uint32_t ns,
-                                            const float* __restrict__ scratch, float* f_s, float* ml_s) {
-  constexpr uint32_t W = D + 2;
-  constexpr uint32_t kCh = 32;  // splits per pass
+                                            const float* __restrict__ scratch, float* f_s) {
+  constexpr uint32_t kCh = 32;  // splits
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t outs = head_rows * D;
   auto row_head = [&](uint32_t hh) __attribute__((always_inline)) {
     return size_t(hh / a.group) * a.q_heads + kv * a.group + hh % a.group;
   };
-  // Common case (<= 32 splits, one output per thread; the packed partial
-  // layout): straight-line code that requests every operand at once -- the
-  // wave's (m_j, l_j) and the thread's 32 numerators, split indices clamped
-  // instead of branched on -- so the merge costs one memory round trip.  The
-  // 64 outputs of a wave lie in one head-row (64 divides D), so every wave
-  // turns its own head-row's (m_j, l_j) into the factors e^{m_j - M} (lane j
-  // holds split j) and reads them back with readlane: no LDS exchange and no
-  // work-group barrier.
-  if (short_merge<D, NW>(ns, head_rows)) {
-    static_assert(D % 64 == 0, "a wave's outputs lie in one head-row");
-    static_assert(kCh == 32, "the short merge covers 32 splits");
-    if (64u * wave >= outs) return;
-    const uint32_t jmax = ns - 1u;
-    const uint32_t hh = (64u * wave) / D;
-    const PackedPartials<D> pp(const_cast<float*>(scratch), a);
-    const size_t rhh = row_head(hh);
-    const uint32_t jl = lane < ns ? lane : jmax;
-    const float mj = ld_agent(pp.m(rhh, a.splits, jl));
-    const float lj = ld_agent(pp.l(rhh, a.splits, jl));
-    const uint32_t d = tid % D;
-    // Numerator j of column d through one descriptor over the head-row's
-    // numerator rows, with the row offset in the instruction's scalar offset
-    // (no per-load vector address arithmetic); agent-coherent cache policy.
-    // Rows past ns - 1 re-read row ns - 1 and are masked below.
-    const float* nb = pp.n(rhh, a.splits, 0) + d;
-    float pre[kCh];
+  static_assert(D % 64 == 0, "a wave's outputs lie in one head-row");
+  static_assert(kCh == 32, "the short merge covers 32 splits");
+  if (64u * wave >= outs) return;
+  const uint32_t jmax = ns - 1u;
+  const uint32_t hh = (64u * wave) / D;
+  const PackedPartials<D> pp(const_cast<float*>(scratch), a);
+  const size_t rhh = row_head(hh);
+  const uint32_t jl = lane < ns ? lane : jmax;
+  const float mj = ld_agent(pp.m(rhh, a.splits, jl));
+  const float lj = ld_agent(pp.l(rhh, a.splits, jl));
+  const uint32_t d = tid % D;
+  // Numerator j of column d through one descriptor over the head-row's
+  // numerator rows, with the row offset in the instruction's scalar offset
+  // (no per-load vector address arithmetic); agent-coherent cache policy.
+  // Rows past ns - 1 re-read row ns - 1 and are masked below.
+  const float* nb = pp.n(rhh, a.splits, 0) + d;
+  float pre[kCh];
 #pragma unroll
-    for (uint32_t j = 0; j < kCh; ++j) pre[j] = ld_agent(nb + size_t(j < jmax ? j : jmax) * D);
-    const bool in = lane < ns;
-    const float mx = wave_max(in ? mj : neg_inf());
-    const float f = in && lj > 0.f ? exp_e(mj - mx) : 0.f;
-    const float lsum = wave_sum(f * lj);
-    // The factors reach every lane as LDS broadcasts (this wave's own 32
-    // floats of f_s), and the 32 products go into four interleaved sums
-    // added as (s0 + s1) + (s2 + s3): a fixed order, four times shorter
-    // dependency chains.
-    float* const fw = f_s + wave * kCh;
-    if (lane < kCh) fw[lane] = f;
-    float fv[kCh];
+  for (uint32_t j = 0; j < kCh; ++j) pre[j] = ld_agent(nb + size_t(j < jmax ? j : jmax) * D);
+  const bool in = lane < ns;
+  const float mx = wave_max(in ? mj : neg_inf());
+  const float f = in && lj > 0.f ? exp_e(mj - mx) : 0.f;
+  const float lsum = wave_sum(f * lj);
+  // The factors reach every lane as LDS broadcasts (this wave's own 32
+  // floats of f_s), and the 32 products go into four interleaved sums
+  // added as (s0 + s1) + (s2 + s3): a fixed order, four times shorter
+  // dependency chains.
+  float* const fw = f_s + wave * kCh;
+  if (lane < kCh) fw[lane] = f;
+  float fv[kCh];
 #pragma unroll
-    for (uint32_t q4 = 0; q4 < kCh / 4u; ++q4) {
-      const float4 x = reinterpret_cast<const float4*>(fw)[q4];
-      fv[4 * q4] = x.x;
-      fv[4 * q4 + 1] = x.y;
-      fv[4 * q4 + 2] = x.z;
-      fv[4 * q4 + 3] = x.w;
-    }
-    float s4[4] = {0.f, 0.f, 0.f, 0.f};
-    if (ns == kCh) {
-#pragma unroll
-      for (uint32_t j = 0; j < kCh; ++j) s4[j & 3u] = fmaf(fv[j], pre[j], s4[j & 3u]);
-    } else {
-#pragma unroll
-      for (uint32_t j = 0; j < kCh; ++j) s4[j & 3u] = fmaf(fv[j], j <= jmax ? pre[j] : 0.f, s4[j & 3u]);
-    }
-    const float nacc = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-    const size_t rh = row_head(hh);
-    if (d == 0) {
-      a.m[rh] = mx;
-      a.l[rh] = lsum;
-    }
-    a.n[rh * D + d] = nacc;
-    if (a.out_type != 0) {
-      const float ov = lsum > 0.f ? nacc / lsum : 0.f;
-      if (a.out_type == 1) static_cast<float*>(a.out)[rh * D + d] = ov;
-      else static_cast<_Float16*>(a.out)[rh * D + d] = (_Float16)ov;
-    }
-    return;
+  for (uint32_t q4 = 0; q4 < kCh / 4u; ++q4) {
+    const float4 x = reinterpret_cast<const float4*>(fw)[q4];
+    fv[4 * q4] = x.x;
+    fv[4 * q4 + 1] = x.y;
+    fv[4 * q4 + 2] = x.z;
+    fv[4 * q4 + 3] = x.w;
   }
-  // Otherwise, where a thread can own four columns of a head-row: merge_rows
-  // (16-byte agent-coherent loads by split groups, one round trip per pass).
-  if constexpr (uint32_t(HS) * D / 4u <= 64u * NW) {
-    merge_rows<D, NW, HS, true>(
-        head_rows, ns, [&](uint32_t hh) { return scratch + row_head(hh) * a.splits * W; }, f_s,
-        [&](uint32_t hh, uint32_t q, float4 nv, float mv, float lv) {
-          const size_t rh = row_head(hh);
-          if (q == 0) {
-            a.m[rh] = mv;
-            a.l[rh] = lv;
-          }
-          float* const nd = a.n + rh * D + 4u * q;  // caller buffers need only 4-byte alignment
-          nd[0] = nv.x;
-          nd[1] = nv.y;
-          nd[2] = nv.z;
-          nd[3] = nv.w;
-          if (a.out_type != 0) {
-            const float o[4] = {lv > 0.f ? nv.x / lv : 0.f, lv > 0.f ? nv.y / lv : 0.f,
-                                lv > 0.f ? nv.z / lv : 0.f, lv > 0.f ? nv.w / lv : 0.f};
-            if (a.out_type == 1) {
-              float* const od = static_cast<float*>(a.out) + rh * D + 4u * q;
-              for (int i = 0; i < 4; ++i) od[i] = o[i];
-            } else {
-              _Float16* const oh = static_cast<_Float16*>(a.out) + rh * D + 4u * q;
-              for (int i = 0; i < 4; ++i) oh[i] = (_Float16)o[i];
-            }
-          }
-        });
-    return;
+  float s4[4] = {0.f, 0.f, 0.f, 0.f};
+  if (ns == kCh) {
+#pragma unroll
+    for (uint32_t j = 0; j < kCh; ++j) s4[j & 3u] = fmaf(fv[j], pre[j], s4[j & 3u]);
+  } else {
+#pragma unroll
+    for (uint32_t j = 0; j < kCh; ++j) s4[j & 3u] = fmaf(fv[j], j <= jmax ? pre[j] : 0.f, s4[j & 3u]);
   }
-  // General case: passes of 32 splits; the running numerator goes through n.
-  for (uint32_t j0 = 0; j0 < ns; j0 += kCh) {
-    const uint32_t cnt = ns - j0 < kCh ? ns - j0 : kCh;
-    for (uint32_t hh = wave; hh < head_rows; hh += NW) {
-      const float* base = scratch + row_head(hh) * a.splits * W;
-      const bool in = lane < cnt;  // lanes >= 32 idle
-      const float mj = in ? ld_agent(base + size_t(j0 + lane) * W) : neg_inf();
-      const float lj = in ? ld_agent(base + size_t(j0 + lane) * W + 1) : 0.f;
-      float mx;
-      if (j0 == 0) {  // M over every split (later passes reuse it)
-        mx = mj;
-        for (uint32_t j = kCh + lane; j < ns; j += 64u) mx = fmaxf(mx, ld_agent(base + size_t(j) * W));
-        mx = wave_max(mx);
-      } else {
-        mx = ml_s[2 * hh];
-      }
-      const float f = lj > 0.f ? exp_e(mj - mx) : 0.f;
-      const float lsum = wave_sum(f * lj);
-      if (lane < kCh) f_s[hh * kCh + lane] = f;
-      if (lane == 0) {
-        ml_s[2 * hh] = mx;
-        ml_s[2 * hh + 1] = (j0 == 0 ? 0.f : ml_s[2 * hh + 1]) + lsum;
-      }
-    }
-    __syncthreads();
-    for (uint32_t idx = tid; idx < outs; idx += 64u * NW) {
-      const uint32_t hh = idx / D, d = idx % D;
-      const float* fh = f_s + hh * kCh;
-      const size_t rh = row_head(hh);
-      float nacc = 0.f;
-      {
-        const float* base = scratch + rh * a.splits * W + 2 + d;
-        const uint32_t jm = j0 + cnt - 1u;
-        float nv[kCh];
-#pragma unroll
-        for (uint32_t j = 0; j < kCh; ++j) nv[j] = ld_agent(base + size_t(j0 + j < jm ? j0 + j : jm) * W);
-        if (j0 != 0) nacc = a.n[rh * D + d];
-#pragma unroll
-        for (uint32_t j = 0; j < kCh; ++j) nacc = fmaf(fh[j], j < cnt ? nv[j] : 0.f, nacc);
-      }
-      if (j0 + kCh < ns) {
-        a.n[rh * D + d] = nacc;  // running numerator, re-read by this thread next pass
-        continue;
-      }
-      const float lsum = ml_s[2 * hh + 1];
-      if (d == 0) {
-        a.m[rh] = ml_s[2 * hh];
-        a.l[rh] = lsum;
-      }
-      a.n[rh * D + d] = nacc;
-      if (a.out_type != 0) {
-        const float o = lsum > 0.f ? nacc / lsum : 0.f;
-        if (a.out_type == 1) static_cast<float*>(a.out)[rh * D + d] = o;
-        else static_cast<_Float16*>(a.out)[rh * D + d] = (_Float16)o;
-      }
-    }
-    __syncthreads();
+  const float nacc = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+  const size_t rh = row_head(hh);
+  if (d == 0) {
+    a.m[rh] = mx;
+    a.l[rh] = lsum;
+  }
+  a.n[rh * D + d] = nacc;
+  if (a.out_type != 0) {
+    const float ov = lsum > 0.f ? nacc / lsum : 0.f;
+    if (a.out_type == 1) static_cast<float*>(a.out)[rh * D + d] = ov;
+    else static_cast<_Float16*>(a.out)[rh * D + d] = (_Float16)ov;
   }
 }
 
@@ -463,6 +360,7 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
   const int64_t* __restrict__ kpos = VARLEN ? a.k_positions : kpos_in;
   const uint32_t* __restrict__ table = VARLEN ? a.page_table : table_in;
   float* __restrict__ scratch = VARLEN ? a.scratch : scratch_in;
+  constexpr int CH = NB == 1 ? 1 : 4;  // tiles per two-pass chunk
   using L = I8Layout<D, NW, HS>;
   constexpr int NC = L::NC;  // MFMA column tiles of the digit columns (PV; QK unless PAIR)
   // Paired-row QK (dim 128, <= 4 head-rows): MFMA row m of M-block mb is
@@ -610,24 +508,26 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
   }
 
   // ---- the wave's tiles (round-robin over the work-group).  Items run in
-  // chunks of 2*kChunk: K images of tiles 4c..4c+3, then their V images.
+  // chunks of 2*CH: K images of tiles 4c..4c+3, then their V images.
   // Items of tiles past the wave's last tile load nothing (zero-sized
   // descriptors); their stale slot contents are masked by tok_ok and zero
   // weights.
   const uint32_t k_vis = e_max > s0 ? (e_max - 1u) / kTileTokens : 0u;
   const uint32_t k_count = e_max > s0 ? k_vis + 1u - k_first : 0u;
   const uint32_t nt = k_count > wave ? (k_count - wave + NW - 1u) / NW : 0u;
-  const uint32_t n_chunks = (nt + kChunk - 1u) / kChunk;
+  const uint32_t n_chunks = (nt + CH - 1u) / CH;
   auto tile_k = [&](uint32_t i) __attribute__((always_inline)) { return k_first + wave + i * NW; };
-  // Item at chunk position POS (0 .. 2*kChunk-1) of chunk ch.
+  // Item at chunk position POS (0 .. 2*CH-1) of chunk ch.
   auto issue = [&](auto posc, uint32_t ch, Slot<D>& slot) __attribute__((always_inline)) {
     constexpr uint32_t pos = decltype(posc)::value;
-    const uint32_t i = ch * kChunk + pos % kChunk;
-    issue_item<D, PT, (pos >= uint32_t(kChunk)), PAIR>(c, tile_k(i), i < nt, slot);
+    const uint32_t i = ch * CH + pos % CH;
+    issue_item<D, PT, (pos >= uint32_t(CH)), PAIR>(c, tile_k(i), i < nt, slot);
   };
-  Slot<D> ring[NB];
+  constexpr int kRing = NB == 1 ? 2 : NB;
+  constexpr int kAhead = NB == 1 ? 2 : NB - 1;
+  Slot<D> ring[kRing];
   // Start streaming before the Q digits are built.
-  static_for<0, NB - 1>([&](auto uc) __attribute__((always_inline)) { issue(uc, 0u, ring[decltype(uc)::value]); });
+  static_for<0, kAhead>([&](auto uc) __attribute__((always_inline)) { issue(uc, 0u, ring[decltype(uc)::value]); });
 
   // ---- Q digits (B operand of QK) and per-head score factors.  A column's
   // scale 2^kq comes from its head-row's whole Q row (with PAIR both tiles
@@ -717,8 +617,8 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
 
   // State.  Lane-as-token view: sc, mx, lw, lrun per head-row.  MFMA view:
   // int32 digit numerators acc_i, fp32 numerators acc_f (head = lane & 15).
-  float sc[kChunk][HS];
-  float vsc[kChunk];  // v-scale of token lane, per tile of the chunk
+  float sc[CH][HS];
+  float vsc[CH];  // v-scale of token lane, per tile of the chunk
   float mx[HS], lw[HS], lrun[HS];
   float m_run[HS], m_new[HS], mu[HS];
   float vmx = 0.f;
@@ -734,7 +634,7 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
     m_new[h] = neg_inf();
     mu[h] = 0.f;
 #pragma unroll
-    for (int r = 0; r < kChunk; ++r) sc[r][h] = neg_inf();
+    for (int r = 0; r < CH; ++r) sc[r][h] = neg_inf();
   }
 #pragma unroll
   for (int mb = 0; mb < D / 16; ++mb) {
@@ -904,22 +804,35 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
     }
   };
 
-  // ---- main loop: one chunk per iteration, items unrolled so that ring
-  // slots (item % NB, NB divides 2*kChunk) are compile-time.
-  static_assert((2 * kChunk) % NB == 0, "ring size must divide the chunk");
-  for (uint32_t ch = 0; ch < n_chunks; ++ch) {
-    static_for<0, 2 * kChunk>([&](auto uc) __attribute__((always_inline)) {
-      constexpr uint32_t u = decltype(uc)::value;
-      issue(std::integral_constant<uint32_t, (u + NB - 1) % (2 * kChunk)>(), ch + (u + NB - 1) / (2 * kChunk),
-            ring[(u + NB - 1) % NB]);
-      if constexpr (u < uint32_t(kChunk)) {
-        process_k(std::integral_constant<uint32_t, u>(), ch * kChunk + u, ring[u % NB]);
-        if constexpr (u == uint32_t(kChunk) - 1) chunk_max();
-      } else {
-        process_v(std::integral_constant<uint32_t, u - kChunk>(), ch * kChunk + (u - kChunk), ring[u % NB]);
-        if constexpr (u == 2u * kChunk - 1) fold();
-      }
-    });
+  if constexpr (NB == 1) {
+    // ---- main loop of one-tile chunks: each slot is refilled as soon as its
+    // item is consumed.
+    for (uint32_t ch = 0; ch < n_chunks; ++ch) {
+      process_k(std::integral_constant<uint32_t, 0>(), ch, ring[0]);
+      chunk_max();
+      issue(std::integral_constant<uint32_t, 0>(), ch + 1u, ring[0]);
+      process_v(std::integral_constant<uint32_t, 0>(), ch, ring[1]);
+      issue(std::integral_constant<uint32_t, 1>(), ch + 1u, ring[1]);
+      fold();
+    }
+  } else {
+    // ---- main loop: one chunk per iteration, items unrolled so that ring
+    // slots (item % NB, NB divides 2*CH) are compile-time.
+    static_assert((2 * CH) % kRing == 0, "ring size must divide the chunk");
+    for (uint32_t ch = 0; ch < n_chunks; ++ch) {
+      static_for<0, 2 * CH>([&](auto uc) __attribute__((always_inline)) {
+        constexpr uint32_t u = decltype(uc)::value;
+        issue(std::integral_constant<uint32_t, (u + NB - 1) % (2 * CH)>(), ch + (u + NB - 1) / (2 * CH),
+              ring[(u + NB - 1) % NB]);
+        if constexpr (u < uint32_t(CH)) {
+          process_k(std::integral_constant<uint32_t, u>(), ch * CH + u, ring[u % NB]);
+          if constexpr (u == uint32_t(CH) - 1) chunk_max();
+        } else {
+          process_v(std::integral_constant<uint32_t, u - CH>(), ch * CH + (u - CH), ring[u % NB]);
+          if constexpr (u == 2u * CH - 1) fold();
+        }
+      });
+    }
   }
 
   // ---- combine the waves through LDS and write the split partial.  Each
@@ -984,16 +897,12 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
     const uint32_t row2 = hh / a.group, head2 = kv * a.group + hh % a.group;
     const size_t rh = size_t(row2) * a.q_heads + head2;
     float* const dst = scratch + (rh * a.splits + split) * W;
-    if constexpr (FUSED) {  // agent-coherent; the short merge's packed layout or the rows
-      const bool packed = short_merge<D, NW>(nsplit, head_rows);
+    if constexpr (FUSED) {  // agent-coherent, in the merge's packed layout
       const PackedPartials<D> pp(scratch, a);
-      float* const pn = packed ? pp.n(rh, a.splits, split) : dst + 2;
-      float* const pm = packed ? pp.m(rh, a.splits, split) : dst;
-      float* const pl = packed ? pp.l(rh, a.splits, split) : dst + 1;
-      __hip_atomic_store(pn + d, val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(pp.n(rh, a.splits, split) + d, val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (d == 0) {
-        __hip_atomic_store(pm, mm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(pl, lsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(pp.m(rh, a.splits, split), mm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(pp.l(rh, a.splits, split), lsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     } else {
       dst[2 + d] = val;
@@ -1023,10 +932,8 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
     __syncthreads();
     if (last_s != 0u) {
       if constexpr (FENCE) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      static_assert(MergeRowsLayout<D, NW, (uint32_t(HS) * D / 4u <= 64u * NW ? HS : 1)>::kFloats * 4u <= L::kBytes,
-                    "the merge's LDS fits the kernel's");
-      float* f_s = reinterpret_cast<float*>(smem);  // [HS][32] split factors or the merge_rows area
-      fused_merge<D, NW, HS>(a, kv, head_rows, nsplit, scratch, f_s, f_s + HS * 32);
+      static_assert(NW * 32 * 4 <= L::kBytes, "the merge's factors fit the kernel's LDS");
+      fused_merge<D, NW>(a, kv, head_rows, nsplit, scratch, reinterpret_cast<float*>(smem));
       if (threadIdx.x == 0) __hip_atomic_store(a.counters + kv, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
@@ -1037,57 +944,77 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
       a.page_tokens, a.kv_heads, a.pages, a, a.q, a.q_positions, a.k_positions, static_cast<const int8_t*>(a.v), \
       a.scratch
 
+// Single-launch instances exist where i8_fusable can choose them.
+template <int NW, int HS>
+constexpr bool kFusedInstance = NW >= 4 && HS <= 4;
+
 template <int D, int NW, int NB, int HS>
 hipError_t launch_cfg(const SplitArgs& a, hipStream_t stream) {
   const bool pt = a.page_tokens >= kTileTokens, fused = a.counters != nullptr, varlen = a.seq_starts != nullptr;
   const dim3 grid(a.splits, a.kv_heads, varlen ? a.batch : 1u);
   const dim3 block(64 * NW);
   if (varlen && !pt) return hipErrorInvalidValue;  // batched calls need whole-tile pages (i8_supported)
-  if (varlen && fused)
-    hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, true, HS, true, true, false>), grid, block, 0, stream, KVB_I8_ARGS);
-  else if (varlen)
+  if (fused) {
+    if constexpr (kFusedInstance<NW, HS>) {
+      if (varlen)
+        hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, true, HS, true, true, false>), grid, block, 0, stream, KVB_I8_ARGS);
+      else if (pt)
+        hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, true, HS, true, false, false>), grid, block, 0, stream, KVB_I8_ARGS);
+      else
+        hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, false, HS, true, false, false>), grid, block, 0, stream, KVB_I8_ARGS);
+      return hipGetLastError();
+    } else {
+      return hipErrorInvalidValue;
+    }
+  }
+  if (varlen)
     hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, true, HS, false, true, false>), grid, block, 0, stream, KVB_I8_ARGS);
-  else if (pt && fused)
-    hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, true, HS, true, false, false>), grid, block, 0, stream, KVB_I8_ARGS);
   else if (pt)
     hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, true, HS, false, false, false>), grid, block, 0, stream, KVB_I8_ARGS);
-  else if (fused)
-    hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, false, HS, true, false, false>), grid, block, 0, stream, KVB_I8_ARGS);
   else
     hipLaunchKernelGGL((split_i8_kernel<D, NW, NB, false, HS, false, false, false>), grid, block, 0, stream, KVB_I8_ARGS);
   return hipGetLastError();
+}
+
+inline hipError_t preload_fns(const void* const* fns, int count) {
+  hipFuncAttributes attr{};
+  for (int i = 0; i < count; ++i) {
+    const hipError_t e = hipFuncGetAttributes(&attr, fns[i]);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 template <int D, int NW, int NB, int HS>
 hipError_t preload_cfg() {
   const void* fns[] = {reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, true, HS, false, false, false>),
                        reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, false, HS, false, false, false>),
-                       reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, true, HS, true, false, false>),
-                       reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, false, HS, true, false, false>),
-                       reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, true, HS, false, true, false>),
-                       reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, true, HS, true, true, false>)};
-  hipFuncAttributes attr{};
-  for (const void* f : fns) {
-    const hipError_t e = hipFuncGetAttributes(&attr, f);
-    if (e != hipSuccess) return e;
+                       reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, true, HS, false, true, false>)};
+  hipError_t e = preload_fns(fns, 3);
+  if constexpr (kFusedInstance<NW, HS>) {
+    const void* one[] = {reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, true, HS, true, false, false>),
+                         reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, false, HS, true, false, false>),
+                         reinterpret_cast<const void*>(&split_i8_kernel<D, NW, NB, true, HS, true, true, false>)};
+    if (e == hipSuccess) e = preload_fns(one, 3);
   }
-  return hipSuccess;
+  return e;
 }
 
 // Launch / preload of every (waves, ring) configuration of one dim; cfg =
-// 10 * waves + ring slots (82 only for head_rows <= 4 and dim <= 128).
+// 10 * waves + ring slots (82 and 81 only for head_rows <= 4 and dim <= 128).
 template <int D>
 hipError_t launch_dim(const SplitArgs& a, int cfg, hipStream_t stream) {
   if (a.rows * a.group <= 4) {
     if constexpr (D <= 128) {
       if (cfg == 82) return launch_cfg<D, 8, 2, 4>(a, stream);
-      if (cfg == 44) return launch_cfg<D, 4, 4, 4>(a, stream);
+      if (cfg == 81) return launch_cfg<D, 8, 1, 4>(a, stream);
     }
+    if (cfg == 41) return launch_cfg<D, 4, 1, 4>(a, stream);
     if (cfg == 12) return launch_cfg<D, 1, 2, 4>(a, stream);
-    if (cfg == 14) return launch_cfg<D, 1, 4, 4>(a, stream);
     return cfg == 42 ? launch_cfg<D, 4, 2, 4>(a, stream) : launch_cfg<D, 2, 2, 4>(a, stream);
   }
   if constexpr (D <= 128) {
+    if (cfg == 41) return launch_cfg<D, 4, 1, 8>(a, stream);
     if (cfg == 12) return launch_cfg<D, 1, 2, 8>(a, stream);
     return cfg == 42 ? launch_cfg<D, 4, 2, 8>(a, stream) : launch_cfg<D, 2, 2, 8>(a, stream);
   }
@@ -1098,18 +1025,17 @@ template <int D>
 hipError_t preload_dim() {
   hipError_t e = hipSuccess;
   if constexpr (D <= 128) {
-    if (e == hipSuccess) e = preload_cfg<D, 8, 2, 4>();
-    if (e == hipSuccess) e = preload_cfg<D, 4, 4, 4>();
+    e = preload_cfg<D, 8, 2, 4>();
+    if (e == hipSuccess) e = preload_cfg<D, 8, 1, 4>();
+    if (e == hipSuccess) e = preload_cfg<D, 4, 1, 8>();
     if (e == hipSuccess) e = preload_cfg<D, 4, 2, 8>();
     if (e == hipSuccess) e = preload_cfg<D, 2, 2, 8>();
+    if (e == hipSuccess) e = preload_cfg<D, 1, 2, 8>();
   }
+  if (e == hipSuccess) e = preload_cfg<D, 4, 1, 4>();
   if (e == hipSuccess) e = preload_cfg<D, 4, 2, 4>();
   if (e == hipSuccess) e = preload_cfg<D, 2, 2, 4>();
   if (e == hipSuccess) e = preload_cfg<D, 1, 2, 4>();
-  if (e == hipSuccess) e = preload_cfg<D, 1, 4, 4>();
-  if constexpr (D <= 128) {
-    if (e == hipSuccess) e = preload_cfg<D, 1, 2, 8>();
-  }
   return e;
 }
 

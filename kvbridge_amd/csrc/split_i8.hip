@@ -19,23 +19,38 @@ namespace {
 
 constexpr uint32_t kTiles = 64;  // tokens per tile
 
-// (waves, ring slots) per work-group as 10 * NW + NB.  A grid of at most
-// two work-groups per CU of a 256-CU device: eight waves (two per SIMD,
-// <= 256 registers each) where the state fits (head_rows <= 4, dim <= 128)
-// and the split has >= 16 tiles.  Larger grids (batches) run several rounds
-// of work-groups per CU, and smaller work-groups that share a CU hide each
-// other's prologue and combine: four waves (two per SIMD) for <= 4
-// head-rows, two waves for 8 head-rows (whose state takes one SIMD per
-// wave).  Measured on MI355X (configs[2] / configs[3] batched calls,
-// 2048-work-group grids): 118 / 216 us with these against 140 / 242 us with
-// the single-sequence choice.  Large grids of short splits (<= 32 tiles)
-// run one wave per work-group: the wave streams its split alone, so there is
-// no wave combine, no work-group barrier and no idle wave per split, and
-// eight such work-groups share a CU.  Measured: cfg2 through launch_attention
+// (waves, ring slots) per work-group as 10 * NW + NB; NB = 1: one-tile chunks.
+//
+// A grid of at most two work-groups per CU of a 256-CU device is bound by
+// the latency of its work-groups when its splits are short: a wave that holds
+// one tile runs a chunk of one (NB = 1) instead of four items of K and of V,
+// three of them empty, and both of its items are in flight from the start.
+// Measured (us per call, graph replay, two launches; dim 128, 4 head-rows
+// unless noted), chunks of four -> of one:
+//   4-tile splits   8,192 tokens 12.96 -> 10.38, 2,048 tokens 12.74 -> 9.83
+//   8-tile splits   4,096 tokens 12.79 -> 12.04 (eight waves)
+//   16-tile splits  32,768 tokens 18.87 -> 18.38 (eight waves)
+//   32-tile splits  65,536 tokens 26.47 -> 27.80: chunks of four stay
+//   8 head-rows     4 tiles 18.32 -> 14.29, 8 tiles 18.50 -> 18.10, 16 tiles 20.37 -> 24.46
+//   dim 256         4 tiles 18.51 -> 15.21, 8 tiles 20.36 -> 19.63
+// Eight waves (two per SIMD, <= 256 registers each) where the state fits
+// (head_rows <= 4, dim <= 128) and the split has more than four tiles; else
+// four.
+//
+// Larger grids (batches) run several rounds of work-groups per CU, and
+// smaller work-groups that share a CU hide each other's prologue and
+// combine: four waves (two per SIMD) for <= 4 head-rows, two waves for 8
+// head-rows (whose state takes one SIMD per wave).  Measured on MI355X (16
+// ragged sequences of 1K .. 32K tokens / 4 sequences of 128K tokens, 8
+// head-rows): 118 / 216 us with these against 140 / 242 us with the
+// single-sequence choice.  Large grids of short splits (<= 32 tiles) run one
+// wave per work-group: the wave streams its split alone, so there is no wave
+// combine, no work-group barrier and no idle wave per split, and eight such
+// work-groups share a CU.  Measured: 65,536 tokens through launch_attention
 // (its 256-token splits, 2,048 work-groups) 47.7 -> 25.3 us for the split
-// launch, configs[3] (64 chunks of 2,048 tokens, 8 head-rows) 203.5 -> 190.6
-// us; configs[2] at 5,120-token splits (80 tiles) stays on four waves (91
-// against 111 us).
+// launch, 4 x 128K tokens (64 chunks of 2,048 tokens, 8 head-rows) 203.5 ->
+// 190.6 us; the ragged batch at 5,120-token splits (80 tiles) stays on four
+// waves (91 against 111 us).
 // KVB_I8_CFG="NW,NB" overrides (tuning sweeps; unknown pairs fall back).
 int i8_config(const SplitArgs& a) {
   static const int forced = [] {
@@ -45,19 +60,18 @@ int i8_config(const SplitArgs& a) {
     if (!e || std::sscanf(e, "%d,%d%c", &nw, &nb, &tail) != 2 || nw < 1 || nw > 9 || nb < 1 || nb > 9) return 0;
     return nw * 10 + nb;
   }();
-  const uint32_t tiles = (a.split_tokens + kTiles - 1) / kTiles;
+  const uint32_t tiles = (a.split_tokens - 1u) / kTiles + 1u;
   const uint32_t hr = a.rows * a.group;
   const bool eight = hr <= 4 && a.dim <= 128;
-  if (forced == 42 || forced == 22 || forced == 12 || ((forced == 82 || forced == 44) && eight) ||
-      (forced == 14 && hr <= 4))
+  if (forced == 42 || forced == 41 || forced == 22 || forced == 12 || ((forced == 82 || forced == 81) && eight))
     return forced;
   const uint64_t groups = uint64_t(a.splits) * a.kv_heads * (a.seq_starts ? a.batch : 1u);
   if (groups > 512u) {
     if (tiles <= 32u) return 12;
     return hr <= 4 ? 42 : 22;
   }
-  if (eight && tiles >= 16) return 82;
-  return tiles >= 4 ? 42 : 22;
+  if (eight) return tiles <= 4 ? 41 : (tiles < 16 ? 81 : 82);
+  return tiles <= 8 ? 41 : 42;
 }
 
 }  // namespace
@@ -74,24 +88,27 @@ bool i8_supported(const SplitArgs& a) {
   return true;
 }
 
-// The in-kernel merge of the single launch is worth it where it is short:
-// the straight-line path (<= 32 splits, a thread per output, a wave per
-// head-row) or at most two merge_rows passes with a thread per four columns;
-// larger merges (e.g. 8 head-rows on two-wave work-groups) run faster as the
-// stand-alone merge kernel, whose work-groups spread over every CU.  Grids
-// of more than two work-groups per CU (batches) also run two launches: every
-// work-group's ticket and the merges then sit between rounds of split work
-// (configs[2]: 116 us for two launches against 121-123 us for one).
+// Whether the single launch runs its in-kernel merge or the call is two
+// launches.  The merge is one work-group per kv head with a thread per output
+// and a wave per head-row, at most 32 splits (otherwise the stand-alone merge,
+// whose work-groups spread over every CU, is faster: 8 head-rows, 32 splits
+// 14.3 against 21.5 us per call, 64 splits 8.5 against 11.0).  Short splits
+// leave the tickets and the merge nothing to hide behind, so below 16 tiles
+// only small grids keep it (us per call, single launch against two):
+//   64 work-groups, 4 x 64 outputs, 4 tiles  7.6 / 8.2;  256, 1 x 128  11.0 / 10.0
+//   64 work-groups, 4 x 128 outputs, 8 tiles 11.4 / 12.0;  4 tiles 10.5 / 9.8
+//   256 work-groups, 1 x 128, 16 tiles 17.5 / 18.4
+// Grids of more than two work-groups per CU (batches) also run two launches:
+// every work-group's ticket and the merges then sit between rounds of split
+// work (16 ragged sequences: 116 us for two launches against 121-123 us).
 bool i8_fusable(const SplitArgs& a) {
   if (!i8_supported(a)) return false;
-  if (uint64_t(a.splits) * a.kv_heads * (a.seq_starts ? a.batch : 1u) > 512u) return false;
-  const uint32_t nw = uint32_t(i8_config(a)) / 10u, threads = 64u * nw;
-  const uint32_t hr = a.rows * a.group, hs = hr <= 4 ? 4u : 8u;
-  if (a.splits <= 32 && hr * a.dim <= threads && hr <= nw) return true;
-  const uint32_t quads = hs * a.dim / 4u;
-  if (quads > threads) return false;
-  const uint32_t groups = threads / quads, per_pass = groups * (groups >= 4 ? 64u / groups : 16u);
-  return (a.splits + per_pass - 1u) / per_pass <= 2u;
+  const uint64_t groups = uint64_t(a.splits) * a.kv_heads * (a.seq_starts ? a.batch : 1u);
+  if (groups > 512u || a.splits > 32u) return false;
+  const uint32_t nw = uint32_t(i8_config(a)) / 10u, hr = a.rows * a.group, outputs = hr * a.dim;
+  if (nw < 4u || hr > nw || outputs > 64u * nw) return false;
+  const uint32_t tiles = (a.split_tokens - 1u) / kTiles + 1u;
+  return tiles >= 16u || (groups <= 128u && (outputs <= 256u || tiles >= 8u));
 }
 
 hipError_t launch_i8_fenced_d128(const SplitArgs& a, hipStream_t stream);
