@@ -133,6 +133,7 @@ kvb::SplitArgs batch_split_args(const kvbridge::BatchShape& b, const kvb_batch_i
   a.total_tokens = b.total_tokens;
   a.table_entries = b.table_entries;
   a.max_tokens = b.max_tokens;
+  a.packed = b.batch <= 256u && uint64_t(a.splits) * a.kv_heads * b.batch > 256u ? 1u : 0u;
   return a;
 }
 

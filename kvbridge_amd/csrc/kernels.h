@@ -46,6 +46,7 @@ struct SplitArgs {
   uint32_t total_tokens;         // k_positions entries (device indices are clamped to it)
   uint32_t table_entries;        // page_table entries (likewise)
   uint32_t max_tokens;           // bound on every sequence's token count
+  uint32_t packed;               // work-groups take live splits first (batch_item, batch.h)
 };
 
 // Sets the thread-local message kvb_last_error() returns; returns code.

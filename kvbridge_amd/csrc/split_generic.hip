@@ -26,7 +26,7 @@ constexpr int kThreads = 256;
 
 template <bool kInt8, bool VARLEN>
 __global__ __launch_bounds__(kThreads) void split_generic_kernel(SplitArgs a) {
-  if constexpr (VARLEN) rebase_sequence(a, blockIdx.z);
+  if constexpr (VARLEN) rebase_sequence(a, blockIdx.z, seq_extent(a, blockIdx.z));
   __shared__ GenericLds<kThreads> lds;
   split_generic_row<kInt8, kThreads>(a, blockIdx.x, blockIdx.y, lds);
 }

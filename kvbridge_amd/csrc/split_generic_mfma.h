@@ -312,7 +312,8 @@ __device__ __forceinline__ uint32_t wave_tiles(const SplitRange& s, uint32_t e_m
   return last < s.first ? 0u : (last - s.first) / s.step + 1u;
 }
 
-// Grid: x = kv head + kv_heads * head-row block, y = split, z = sequence.
+// Grid: x = kv head + kv_heads * head-row block, y = split, z = sequence (see
+// batch_item).
 //
 // int8 KV.  MFMA row m of QK M-block mb is token 16 (m / 4) + 4 mb + m % 4 of
 // the 64-token tile, so lane (n, g) ends up with the scores of tokens 16g ..
@@ -323,13 +324,18 @@ __device__ __forceinline__ uint32_t wave_tiles(const SplitRange& s, uint32_t e_m
 template <int DP, int NW, bool VARLEN>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(DP <= 128 ? 2 : 1)))
 void split_generic_i8_kernel(SplitArgs a) {
-  if constexpr (VARLEN) rebase_sequence(a, blockIdx.z);
+  uint32_t split = blockIdx.y;
+  if constexpr (VARLEN) {
+    const BatchItem item = batch_item(a);
+    split = item.split;
+    rebase_sequence(a, item.seq, item.e);
+  }
   __shared__ __attribute__((aligned(16))) GenericSmem<DP, NW> sm;
   constexpr uint32_t TILE = 64;
   constexpr int KS = DP / 64;   // 64-dim steps
   constexpr int MB = DP / 16;   // V row blocks
   const uint32_t lane = threadIdx.x & 63u, n = lane & 15u, g = lane >> 4;
-  const uint32_t kv = blockIdx.x % a.kv_heads, hb = blockIdx.x / a.kv_heads, split = blockIdx.y;
+  const uint32_t kv = blockIdx.x % a.kv_heads, hb = blockIdx.x / a.kv_heads;
   const SplitRange s = split_range<NW>(a, split, TILE);
   if (s.s1 <= s.s0) return write_empty<NW>(a, kv, hb, split);
   OnlineState<DP> st;
@@ -491,12 +497,17 @@ void split_generic_i8_kernel(SplitArgs a) {
 template <int DP, int NW, bool VARLEN>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(DP <= 128 ? 2 : 1)))
 void split_generic_f32_kernel(SplitArgs a) {
-  if constexpr (VARLEN) rebase_sequence(a, blockIdx.z);
+  uint32_t split = blockIdx.y;
+  if constexpr (VARLEN) {
+    const BatchItem item = batch_item(a);
+    split = item.split;
+    rebase_sequence(a, item.seq, item.e);
+  }
   __shared__ __attribute__((aligned(16))) GenericSmem<DP, NW> sm;
   constexpr uint32_t TILE = 16;
   constexpr int MB = DP / 16;  // 16-dim steps of QK, V row blocks
   const uint32_t lane = threadIdx.x & 63u, n = lane & 15u, g = lane >> 4;
-  const uint32_t kv = blockIdx.x % a.kv_heads, hb = blockIdx.x / a.kv_heads, split = blockIdx.y;
+  const uint32_t kv = blockIdx.x % a.kv_heads, hb = blockIdx.x / a.kv_heads;
   const SplitRange s = split_range<NW>(a, split, TILE);
   if (s.s1 <= s.s0) return write_empty<NW>(a, kv, hb, split);
   OnlineState<DP> st;

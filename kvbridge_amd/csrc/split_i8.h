@@ -328,7 +328,8 @@ __device__ __forceinline__ void fused_merge(const SplitArgs& a, uint32_t kv, uin
   }
 }
 
-// VARLEN: batched call, grid.z = sequence (arguments rebased per work-group).
+// VARLEN: batched call, grid (kv heads, splits, sequences) in the order of
+// batch_item (arguments rebased per work-group).
 // The leading scalar arguments are everything the first KV request depends
 // on; the translation units that instantiate this kernel are built with
 // kernel-argument preloading for them (the dispatcher places them in SGPRs),
@@ -354,7 +355,13 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
   a.page_tokens = p_page_tokens;
   a.kv_heads = p_kv_heads;
   a.pages = p_pages;
-  if constexpr (VARLEN) rebase_sequence(a, blockIdx.z);
+  uint32_t split = blockIdx.x, kv = blockIdx.y;
+  if constexpr (VARLEN) {
+    const BatchItem item = batch_item(a);
+    split = item.split;
+    kv = blockIdx.x;
+    rebase_sequence(a, item.seq, item.e);
+  }
   const float* __restrict__ q = VARLEN ? a.q : q_in;
   const int64_t* __restrict__ qpos = VARLEN ? a.q_positions : qpos_in;
   const int64_t* __restrict__ kpos = VARLEN ? a.k_positions : kpos_in;
@@ -376,8 +383,6 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t n = lane & 15u, g = lane >> 4;
-  const uint32_t split = blockIdx.x;
-  const uint32_t kv = blockIdx.y;
   const uint32_t head_rows = a.rows * a.group;  // <= HS
   // Splits that take part in the fused merge.  A batched single-launch call
   // merges only the sequence's own splits (at least one, so that an empty
@@ -951,7 +956,7 @@ constexpr bool kFusedInstance = NW >= 4 && HS <= 4;
 template <int D, int NW, int NB, int HS>
 hipError_t launch_cfg(const SplitArgs& a, hipStream_t stream) {
   const bool pt = a.page_tokens >= kTileTokens, fused = a.counters != nullptr, varlen = a.seq_starts != nullptr;
-  const dim3 grid(a.splits, a.kv_heads, varlen ? a.batch : 1u);
+  const dim3 grid = varlen ? dim3(a.kv_heads, a.splits, a.batch) : dim3(a.splits, a.kv_heads, 1u);  // batch_item
   const dim3 block(64 * NW);
   if (varlen && !pt) return hipErrorInvalidValue;  // batched calls need whole-tile pages (i8_supported)
   if (fused) {
