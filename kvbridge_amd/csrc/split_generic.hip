@@ -3,7 +3,8 @@
 // pages or with many head-rows.  The MFMA kernels (split_generic_mfma.h) serve
 // the shapes they can load in whole 16-byte pieces, the scalar kernel here
 // (split_generic.h) the rest: dims that are not a multiple of 4, pages that
-// are not a multiple of 16 tokens.
+// are not a multiple of 16 tokens.  Dim 128 batches over small pages with few
+// head-rows run the four-digit int8 kernel (split_i8_wide.hip).
 //
 // Scalar kernel: grid x = row * q_heads + head, y = split, z = sequence of a
 // batched call; block of 256 threads (4 waves).
@@ -42,25 +43,29 @@ bool mfma_supported(const SplitArgs& a, bool int8) {
   return a.kv_heads * blocks < (uint64_t(1) << 22);
 }
 
-// Waves per work-group.  Up to two work-groups per CU: as many as the split
-// has tiles for, because a lone work-group is bound by latency (8,000 tokens,
-// dim 96, 128 work-groups of 8 tiles: split kernel 11.5 us with 8 waves,
-// 15.0 with 2).  Larger grids: two waves, so that four work-groups share a CU
-// and hide each other's prologue and combine (32 sequences of 100 .. 4,000
-// tokens, dim 128, 2,048 work-groups: 49 us per call with 2 waves, 51 with 4,
-// 73 with 8).  The state of dims above 128 takes a SIMD per wave.
+// Waves per work-group.  int8 (64-token tiles): four -- more leave a wave one
+// tile and a longer combine, fewer leave the CUs short of requests (us per
+// call, 8 / 4 / 2 waves: dim 96, 8,000 tokens 16.2 / 16.2 / 19.7; 8 ragged
+// sequences of up to 4,000 tokens, 8 head-rows 27.4 / 21.8 / 25.8; the same
+// 32 sequences 69.4 / 47.9 / 48.2); two where several work-groups per CU
+// have only four tiles each (16 sequences, 256-token splits 57.5 / 35.3 /
+// 32.7).  fp32 (16-token tiles): eight where the registers allow it and a
+// work-group has a CU to itself (dim 64, 8,192 tokens 14.4 / 16.6 / 24.4).
 int mfma_waves(const SplitArgs& a, bool int8) {
   const uint32_t tile = int8 ? 64u : 16u, tiles = (a.split_tokens - 1u) / tile + 1u;
   const uint64_t blocks = (uint64_t(a.rows) * a.group + 15u) / 16u;
   const uint64_t groups = blocks * a.kv_heads * a.splits * (a.seq_starts ? a.batch : 1u);
-  int nw = groups > 512u ? 2 : (a.dim <= 128 ? 8 : 4);
-  while (nw > 1 && uint32_t(nw) > tiles) nw /= 2;
-  return nw;
+  uint32_t nw = 4;
+  if (int8 && groups > 1024u && tiles <= 4u) nw = 2;
+  if (!int8 && a.dim <= 128 && groups <= 512u) nw = 8;
+  while (nw > tiles) nw /= 2u;
+  return int(nw);
 }
 
 }  // namespace
 
 hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t stream) {
+  if (int8 && i8_wide_supported(a)) return launch_split_i8_wide(a, stream);
   if (mfma_supported(a, int8)) {
     const int nw = mfma_waves(a, int8);
     return int8 ? launch_generic_i8(a, nw, stream) : launch_generic_f32(a, nw, stream);
@@ -84,7 +89,9 @@ const char* generic_kernel_name(const SplitArgs& a, bool int8) {
   const char* const t = int8 ? "true" : "false";
   const char* const v = a.seq_starts != nullptr ? "true" : "false";
   const int at = std::snprintf(buf, sizeof(buf), "split_generic_kernel<%s, %s>", t, v);
-  if (mfma_supported(a, int8))
+  if (int8 && i8_wide_supported(a))
+    std::snprintf(buf + at, sizeof(buf) - at, ": %s", i8_wide_kernel_name(a));
+  else if (mfma_supported(a, int8))
     std::snprintf(buf + at, sizeof(buf) - at, ": split_generic_%s_kernel<%d, %d, %s>", int8 ? "i8" : "f32",
                   a.dim <= 64 ? 64 : (a.dim <= 128 ? 128 : 256), mfma_waves(a, int8), v);
   return buf;
@@ -100,8 +107,9 @@ hipError_t preload_generic() {
     const hipError_t e = hipFuncGetAttributes(&attr, f);
     if (e != hipSuccess) return e;
   }
-  const hipError_t e = preload_generic_i8();
-  return e != hipSuccess ? e : preload_generic_f32();
+  hipError_t e = preload_generic_i8();
+  if (e == hipSuccess) e = preload_generic_f32();
+  return e == hipSuccess ? preload_i8_wide() : e;
 }
 
 }  // namespace kvb

@@ -15,9 +15,6 @@ hipError_t launch_nw(const SplitArgs& a, hipStream_t stream) {
 
 template <int DP>
 hipError_t launch_dim(const SplitArgs& a, int nw, hipStream_t stream) {
-  if constexpr (DP <= 128) {
-    if (nw == 8) return launch_nw<DP, 8>(a, stream);
-  }
   return nw == 4 ? launch_nw<DP, 4>(a, stream) : (nw == 2 ? launch_nw<DP, 2>(a, stream) : launch_nw<DP, 1>(a, stream));
 }
 
@@ -35,9 +32,6 @@ hipError_t preload_dim() {
   hipError_t e = preload_nw<DP, 1>();
   if (e == hipSuccess) e = preload_nw<DP, 2>();
   if (e == hipSuccess) e = preload_nw<DP, 4>();
-  if constexpr (DP <= 128) {
-    if (e == hipSuccess) e = preload_nw<DP, 8>();
-  }
   return e;
 }
 

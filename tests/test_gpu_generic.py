@@ -142,3 +142,36 @@ def test_non_finite_values_match_the_scalar_kernel(gpu, what, int8):
         log(f"  {what} int8={int8} {nm}: {np.count_nonzero(~fin)} non-finite")
         if fin.any():
             np.testing.assert_allclose(x[fin], y[fin], rtol=5e-5, atol=3e-6 * max(1.0, np.abs(y[fin]).max()))
+
+
+WIDE_BATCHES = [
+    # kv_heads, group, page, lengths, split: one per (waves, ring) choice
+    (8, 4, 16, [300, 0, 1, 1000, 64, 777], 256),          # short splits, small grid
+    (8, 4, 32, [5000, 1024, 2047], 1024),                 # 16 tiles
+    (4, 3, 16, [130, 4000, 33, 0, 64] * 12, 256),         # four tiles, large grid
+    (8, 1, 32, [100, 4000, 1500, 513] * 5, 512),          # eight tiles, large grid
+    (8, 2, 16, [70000, 12], 2112),                        # 33 tiles, page window outrun
+]
+
+
+@pytest.mark.parametrize("cfg", WIDE_BATCHES)
+def test_four_digit_batches(gpu, cfg):
+    """The four-digit kernel is held to fp32 accuracy: error against FP64 at
+    most 1e-6 of each head-row's largest numerator (two fp32 roundings per
+    partial and merge step; weights rounded at 2^-28)."""
+    kvh, group, p, lengths, st = cfg
+    bc = W.synth_batch(1, kvh * group, kvh, 128, p, lengths, seed=kvh * group + p, split_tokens=st)
+    db = DeviceBatch(bc.shape, bc.to_device("cuda:0"))
+    name = kvb.batch_kernel_name(bc.shape, db.inp)
+    log(f"four-digit batch shape={bc.shape.as_tuple()} kernel={name}")
+    assert ": split_i8_wide_kernel<128," in name
+    m, l, n, _ = db.run(fused=False)
+    for b in range(min(6, len(lengths))):
+        g = check_sequence_vs_oracle(bc, b, m, l, n, f"seq {b}")
+        if g is None:
+            continue
+        ref, _ = O.fp64(bc.sequence(b), threads=8)
+        sl = slice(b * kvh * group, (b + 1) * kvh * group)
+        got = n.reshape(-1, 128)[sl].astype(np.float64) / l[sl, None].astype(np.float64)
+        err = np.abs(got - ref.reshape(got.shape)).max(1) / np.abs(ref.reshape(got.shape)).max(1)
+        assert g["strict_pass"] and err.max() <= 1e-6, (b, err.max())
