@@ -119,11 +119,30 @@ def device_input(q, q_positions, k_positions, page_table, k, v, k_scales=None, v
     return DeviceInput(*(_ptr(x) for x in (q, q_positions, k_positions, page_table, k, v, k_scales, v_scales)))
 
 
+_raw_stream = None  # torch's handle-only query, looked up once
+
+
+def _current_stream() -> int:
+    """Handle of torch's current HIP stream on the current device.
+
+    torch.cuda.current_stream() builds a stream object for it, 2.7 us of the
+    7.1 us that a single-launch call took on the host; the query that returns
+    the handle alone takes 0.2 us.  Before torch has initialized the device,
+    and on a torch without that query, the public call serves."""
+    global _raw_stream
+    import torch
+
+    if _raw_stream is None:
+        get, device = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+        _raw_stream = (lambda: get(device())) if get and device else False
+    if _raw_stream and torch.cuda.is_initialized():
+        return _raw_stream()
+    return torch.cuda.current_stream().cuda_stream
+
+
 def _stream(stream) -> int | None:
     if stream is None:
-        import torch
-
-        return torch.cuda.current_stream().cuda_stream
+        return _current_stream()
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
