@@ -47,22 +47,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const float* p, uint
 
 }  // namespace merge_detail
 
-// R <= RM row-heads, S >= 1 splits.  row_base(r) -> const float* (r < R).
+// PAD: dim (a multiple of 4) may be less than D, else it is D.  R <= RM
+// row-heads, S >= 1 splits.  row_base(r) -> const float* (r < R).
 // emit(r, q, N (float4: columns 4q..4q+3), M, L) is called once per quad
 // of every row-head, by the thread that owns it.  lds: kFloats floats,
 // 16-byte aligned.  Every thread of the work-group must call this.
-template <int D, int NW, int RM, typename RowBase, typename Emit>
-__device__ __forceinline__ void merge_rows(uint32_t R, uint32_t S, RowBase row_base, float* lds, Emit emit) {
+template <int D, int NW, int RM, bool PAD, typename RowBase, typename Emit>
+__device__ __forceinline__ void merge_rows(uint32_t dim, uint32_t R, uint32_t S, RowBase row_base, float* lds,
+                                           Emit emit) {
   using L = MergeRowsLayout<D, NW, RM>;
   using merge_detail::u32x4;
-  constexpr uint32_t W = D + 2;
+  const uint32_t W = PAD ? dim + 2u : uint32_t(D) + 2u;
   float* const fs = lds;                                                   // [RM][kPS]
   float* const ml = lds + RM * L::kPS;                                     // [RM][4]: M, L
   float4* const part = reinterpret_cast<float4*>(lds + RM * L::kPS + 4 * RM);  // [kG][kQT]
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t g = tid / L::kQT, e = tid % L::kQT;
   const uint32_t r = e / L::kQ, q = e % L::kQ;
-  const bool mine = g < L::kG && r < R;
+  const bool mine = g < L::kG && r < R && (!PAD || 4u * q < dim);
+  const uint32_t qc = PAD && 4u * q >= dim ? 0u : q;  // a quad past dim loads the first one and drops it
   const uint32_t rr = mine ? r : 0u;
   const __amdgpu_buffer_rsrc_t rs = merge_detail::rows_rsrc(row_base(rr), S * W * 4u);
   const uint32_t passes = (S + L::kPS - 1u) / L::kPS;
@@ -87,7 +90,7 @@ __device__ __forceinline__ void merge_rows(uint32_t R, uint32_t S, RowBase row_b
 #pragma unroll
     for (uint32_t k = 0; k < L::kK; ++k) {
       const uint32_t j = j0 + g + L::kG * k;
-      v[k] = __builtin_amdgcn_raw_buffer_load_b128(rs, int(((j < jmax ? j : jmax) * W + 2u + 4u * q) * 4u), 0, 0);
+      v[k] = __builtin_amdgcn_raw_buffer_load_b128(rs, int(((j < jmax ? j : jmax) * W + 2u + 4u * qc) * 4u), 0, 0);
     }
     for (uint32_t h = wave; h < R; h += NW) {
       const float* b = row_base(h);
@@ -111,7 +114,9 @@ __device__ __forceinline__ void merge_rows(uint32_t R, uint32_t S, RowBase row_b
 #pragma unroll
       for (uint32_t k = 0; k < L::kK; ++k) {
         const uint32_t jl = g + L::kG * k;
-        if (j0 + jl < S) {
+        // Padded dims leave a split of factor 0 out, whatever its numerators
+        // hold (splits of non-finite values reach this merge).
+        if (j0 + jl < S && (!PAD || fr[jl] != 0.f)) {
           const float f = fr[jl];
           acc.x = fmaf(f, __uint_as_float(v[k][0]), acc.x);
           acc.y = fmaf(f, __uint_as_float(v[k][1]), acc.y);
@@ -124,7 +129,7 @@ __device__ __forceinline__ void merge_rows(uint32_t R, uint32_t S, RowBase row_b
   }
   if (g < L::kG) part[g * L::kQT + e] = acc;
   __syncthreads();
-  if (g == 0 && r < R) {
+  if (g == 0 && mine) {
     float4 nsum = part[e];
 #pragma unroll
     for (uint32_t gg = 1; gg < L::kG; ++gg) {

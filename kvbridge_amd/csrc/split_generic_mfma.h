@@ -24,7 +24,7 @@
 // in registers (ring of two) gained nothing (head size 96, 8,000 tokens: 16.9
 // us per call with it, 15.9 without).  Measured per call against one scalar
 // work-group per head-row (32 q / 8 kv heads): dim 96, 8,000 tokens 132 ->
-// 15.9 us; fp32 KV, dim 128, 8,192 tokens 150 -> 25.6 us (16-token tiles on
+// 13.2 us; fp32 KV, dim 128, 8,192 tokens 150 -> 25.6 us (16-token tiles on
 // 128 work-groups, 26 GB/s per CU); 32 sequences of 100 .. 4,000 tokens over
 // 16-token pages, dim 128, 916 -> 49 us.  Error against 64 bits: no larger
 // (n 4.9e-7 / 2.8e-7 / 3.0e-7 relative, 6.9e-7 / 3.6e-7 / 3.9e-7 scalar).
@@ -179,13 +179,16 @@ template <int DP, int NW>
 union GenericSmem {
   u32x4_g q[DP / 64][2][3][64];  // int8: Q pieces of every lane
   struct {
-    float m[NW][16], l[NW][16];
+    float m[NW][16], l[NW][16], f[NW][16];
     float acc[NW][16][DP + 4];  // padded rows: 16 head-rows of one column spread over the banks
   } c;
   GenericLds<64 * NW> scalar;
 };
 
-// Combines the waves (m in log2 units, l summed over the lanes of a head-row
+// Combines the waves (the visible part of a short split: dim 128, 16
+// head-rows, 3.2 of the split kernel's 12.7 us while every thread computed the
+// factors and took one column per step; a quad per thread took 2 us off; m in
+// log2 units, l summed over the lanes of a head-row
 // already) and writes the block's partials; a block with a non-finite result
 // goes through the scalar rows instead.
 template <int DP, int NW, bool kInt8>
@@ -219,28 +222,41 @@ __device__ __forceinline__ void write_partials(const SplitArgs& a, const HeadLan
     }
     return;
   }
-  const uint32_t chunks = (a.dim + 63u) / 64u;
-  for (uint32_t c = wave; c < rows_here * chunks; c += NW) {
-    const uint32_t r = c / chunks, d = (c - r * chunks) * 64u + lane;
-    const bool in = d < a.dim;
-    float mw[NW], mm = neg_inf();
+  // Factors of the waves, one (wave, head-row) per lane of wave 0, then a
+  // quad of columns per thread: independent 16-byte LDS loads and one store.
+  if (tid < 16u * NW) {
+    const uint32_t r = tid & 15u, w = tid >> 4;
+    if (r < rows_here) {
+      float mm = sm.c.m[0][r];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      mw[w] = sm.c.m[w][r];
-      mm = fmaxf(mm, mw[w]);
+      for (int i = 1; i < NW; ++i) mm = fmaxf(mm, sm.c.m[i][r]);
+      const float mw = sm.c.m[w][r];
+      sm.c.f[w][r] = mw == neg_inf() ? 0.f : exp_e(mw - mm);
     }
-    float val = 0.f, ls = 0.f;
+  }
+  __syncthreads();
+  constexpr uint32_t QT = DP / 4;  // threads per head-row
+  const uint32_t q = tid % QT;
+  for (uint32_t r = tid / QT; r < rows_here; r += 64u * NW / QT) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    float ls = 0.f, mm = neg_inf();
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float f = mw[w] == neg_inf() ? 0.f : exp_e(mw[w] - mm);
+      const float f = sm.c.f[w][r];
+      const f32x4 x = *reinterpret_cast<const f32x4*>(&sm.c.acc[w][r][4u * q]);
       ls = fmaf(f, sm.c.l[w][r], ls);
-      val = fmaf(f, sm.c.acc[w][r][in ? d : 0u], val);
+      mm = fmaxf(mm, sm.c.m[w][r]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = fmaf(f, x[e], v[e]);
     }
     const uint32_t hh = 16u * hb + r;
     const size_t rh = size_t(hh / a.group) * a.q_heads + kv * a.group + hh % a.group;
     float* const dst = a.scratch + (rh * a.splits + split) * (size_t(a.dim) + 2);
-    if (in) dst[2u + d] = val;
-    if (d == 0u) {
+    if (4u * q < a.dim) {  // dim is a multiple of 4; partial rows are only 4-byte aligned
+      typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+      *reinterpret_cast<f32x4_u*>(dst + 2u + 4u * q) = v;
+    }
+    if (q == 0u) {
       dst[0] = mm;
       dst[1] = ls;
     }

@@ -144,6 +144,23 @@ def test_non_finite_values_match_the_scalar_kernel(gpu, what, int8):
             np.testing.assert_allclose(x[fin], y[fin], rtol=5e-5, atol=3e-6 * max(1.0, np.abs(y[fin]).max()))
 
 
+@pytest.mark.parametrize("dim,tokens,rows", [(4, 64 * 128, 1), (60, 3 * 128, 1), (68, 17 * 128, 2), (96, 64 * 128, 1),
+                                             (252, 33 * 128, 1), (96, 65 * 128, 1)])
+def test_padded_merge(gpu, dim, tokens, rows):
+    """Merges of dims between the powers of two: 1 .. 64 splits through the
+    padded merge, 65 through the scalar one, the last splits empty; against
+    the oracle's merge of the same partials (fp32, other order of the sums)."""
+    case = W.synth_case(rows, 8, 2, dim, 16, tokens, seed=dim, qpos=[tokens // 2] * rows)
+    dc = DeviceCase(case)
+    (m, l, n), out, sc = dc.run_decode(128)
+    parts = sc.cpu().numpy()
+    m_ref, l_ref, n_ref = O.merge_fp32(case.shape, parts, tokens // 128)
+    assert np.array_equal(m, m_ref)
+    np.testing.assert_allclose(l, l_ref, rtol=1e-5)
+    np.testing.assert_allclose(n, n_ref, rtol=1e-5, atol=1e-5 * np.abs(n_ref).max())
+    np.testing.assert_allclose(out.ravel(), (n.reshape(-1, dim) / l[:, None]).ravel(), rtol=1e-6)
+
+
 WIDE_BATCHES = [
     # kv_heads, group, page, lengths, split: one per (waves, ring) choice
     (8, 4, 16, [300, 0, 1, 1000, 64, 777], 256),          # short splits, small grid
