@@ -32,17 +32,6 @@ __global__ __launch_bounds__(kThreads) void split_generic_kernel(SplitArgs a) {
   split_generic_row<kInt8, kThreads>(a, blockIdx.x, blockIdx.y, lds);
 }
 
-// Shapes of the MFMA kernels: K rows and V columns in dword-aligned 16-byte
-// loads (dim a multiple of 4, whole 16-token groups in a page), fp32 V slabs
-// within 32-bit byte offsets, and a grid of head-row blocks that fits grid.x.
-bool mfma_supported(const SplitArgs& a, bool int8) {
-  if (a.dim % 4 != 0 || a.page_tokens % 16 != 0) return false;
-  if (reinterpret_cast<uintptr_t>(a.k) % 4 != 0 || reinterpret_cast<uintptr_t>(a.v) % 4 != 0) return false;
-  if (!int8 && uint64_t(a.dim) * a.page_tokens >= (uint64_t(1) << 30)) return false;
-  const uint64_t blocks = (uint64_t(a.rows) * a.group + 15u) / 16u;
-  return a.kv_heads * blocks < (uint64_t(1) << 22);
-}
-
 // Waves per work-group.  int8 (64-token tiles): four -- more leave a wave one
 // tile and a longer combine, fewer leave the CUs short of requests (us per
 // call, 8 / 4 / 2 waves: dim 96, 8,000 tokens 16.2 / 16.2 / 19.7; 8 ragged
@@ -64,9 +53,20 @@ int mfma_waves(const SplitArgs& a, bool int8) {
 
 }  // namespace
 
+// Shapes of the MFMA kernels: K rows and V columns in dword-aligned 16-byte
+// loads (dim a multiple of 4, whole 16-token groups in a page), fp32 V slabs
+// within 32-bit byte offsets, and a grid of head-row blocks that fits grid.x.
+bool generic_mfma_supported(const SplitArgs& a, bool int8) {
+  if (a.dim % 4 != 0 || a.page_tokens % 16 != 0) return false;
+  if (reinterpret_cast<uintptr_t>(a.k) % 4 != 0 || reinterpret_cast<uintptr_t>(a.v) % 4 != 0) return false;
+  if (!int8 && uint64_t(a.dim) * a.page_tokens >= (uint64_t(1) << 30)) return false;
+  const uint64_t blocks = (uint64_t(a.rows) * a.group + 15u) / 16u;
+  return a.kv_heads * blocks < (uint64_t(1) << 22);
+}
+
 hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t stream) {
   if (int8 && i8_wide_supported(a)) return launch_split_i8_wide(a, stream);
-  if (mfma_supported(a, int8)) {
+  if (generic_mfma_supported(a, int8)) {
     const int nw = mfma_waves(a, int8);
     return int8 ? launch_generic_i8(a, nw, stream) : launch_generic_f32(a, nw, stream);
   }
@@ -91,7 +91,7 @@ const char* generic_kernel_name(const SplitArgs& a, bool int8) {
   const int at = std::snprintf(buf, sizeof(buf), "split_generic_kernel<%s, %s>", t, v);
   if (int8 && i8_wide_supported(a))
     std::snprintf(buf + at, sizeof(buf) - at, ": %s", i8_wide_kernel_name(a));
-  else if (mfma_supported(a, int8))
+  else if (generic_mfma_supported(a, int8))
     std::snprintf(buf + at, sizeof(buf) - at, ": split_generic_%s_kernel<%d, %d, %s>", int8 ? "i8" : "f32",
                   a.dim <= 64 ? 64 : (a.dim <= 128 ? 128 : 256), mfma_waves(a, int8), v);
   return buf;

@@ -28,6 +28,9 @@ SHAPES = [
     (1, 32, 8, 132, 16, 600, 0, 600, 256, True, None),       # four-wave instances
     (1, 24, 4, 252, 16, 1100, 0, 1100, 1024, True, None),
     (1, 8, 2, 96, 16, 20000, 0, 20000, 20000, True, None),   # one split of 313 tiles: several row windows
+    (3, 24, 8, 128, 64, 1500, 0, 1500, 256, True, [1499, 3, 700]),  # 9 head-rows of a tiled shape
+    (4, 16, 4, 64, 16, 1500, 5, 1490, 320, True, None),      # 16 head-rows, off-tile begin
+    (2, 64, 8, 128, 32, 3000, 0, 3000, 1000, True, None),    # off-tile splits
     (1, 4, 4, 4, 16, 200, 0, 200, 64, False, None),
     (1, 8, 2, 64, 16, 700, 5, 695, 128, False, None),
     (1, 16, 1, 100, 48, 1000, 0, 1000, 256, False, None),
