@@ -139,7 +139,8 @@ kvb::SplitArgs batch_split_args(const kvbridge::BatchShape& b, const kvb_batch_i
 
 // The batched split kernel: int8 MFMA where it applies, else the generic one.
 bool batch_uses_i8(const kvbridge::BatchShape& b, const kvb_batch_input& in, const kvb::SplitArgs& a) {
-  return kvb::tiled_supported(batch_sequence_shape(b), batch_device_input(in)) && kvb::i8_supported(a);
+  return kvb::tiled_supported(batch_sequence_shape(b), batch_device_input(in)) && kvb::i8_supported(a) &&
+         !kvb::one_block_rows(a);
 }
 
 }  // namespace
@@ -186,31 +187,17 @@ static bool force_f16() {
   return f;
 }
 
-// 9 to 16 head-rows (a few query rows of one sequence) at dim 64 and 128, up
-// to two work-groups per CU: the generic MFMA kernel, whose one block of 16
-// columns they fill, streams into registers and keeps four waves on one split,
-// where the rows kernels stage the split through LDS for up to four blocks.
-// Measured (us per call, rows / f16 kernel -> generic): 4 rows x 32 q / 8 kv
-// heads, dim 128, 16,001 tokens in splits of 512 / 1,024 18.2 -> 14.9 / 25.6 ->
-// 19.2, 4,000 tokens in 256 14.8 -> 12.6; dim 64, 16,001 tokens in 512 13.3 ->
-// 10.0.  17 to 32 head-rows are two blocks that each read the KV (19.6 against
-// 22.8 at dim 128, 512-token splits) and stay.
-static bool one_block_rows(const SplitArgs& a) {
-  const uint64_t hr = uint64_t(a.rows) * a.group;
-  return hr > 8u && hr <= 16u && a.dim <= 128u && uint64_t(a.splits) * a.kv_heads <= 512u && generic_mfma_supported(a, true);
-}
-
 hipError_t launch_split_fast(const SplitArgs& a, hipStream_t stream) {
-  if (!force_f16() && i8_supported(a)) return launch_split_i8(a, stream);
   if (!force_f16() && one_block_rows(a)) return launch_split_generic(a, true, stream);
+  if (!force_f16() && i8_supported(a)) return launch_split_i8(a, stream);
   if (!force_f16() && i8_rows_supported(a)) return launch_split_i8_rows(a, stream);
   return launch_split_lds(a, stream);
 }
 
 const char* split_kernel_name(const SplitArgs& a, bool tiled, bool int8) {
   if (!tiled) return generic_kernel_name(a, int8);
-  if (!force_f16() && i8_supported(a)) return i8_kernel_name(a);
   if (!force_f16() && one_block_rows(a)) return generic_kernel_name(a, true);
+  if (!force_f16() && i8_supported(a)) return i8_kernel_name(a);
   if (!force_f16() && i8_rows_supported(a)) return i8_rows_kernel_name(a);
   return lds_kernel_name(a);
 }

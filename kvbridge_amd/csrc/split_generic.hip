@@ -64,6 +64,31 @@ bool generic_mfma_supported(const SplitArgs& a, bool int8) {
   return a.kv_heads * blocks < (uint64_t(1) << 22);
 }
 
+// 5 to 16 head-rows at dim 64 and 128 fill the generic kernel's one block of
+// columns, which costs it the same for any number of them, and its state fits
+// two waves per SIMD.
+//  * 5 to 8 (wide GQA): the int8 kernel's state for 8 head-rows takes a SIMD
+//    per wave.  us per call, int8 -> generic, 64 q / 8 kv heads, dim 128:
+//    splits of 256, 8,192 tokens 14.4 -> 11.3, 65,536 tokens 45.3 -> 40.9; of
+//    512, 16,384 tokens 18.3 -> 14.1; dim 64, 16 q / 2 kv heads 12.6 -> 9.9;
+//    32 sequences of 100 .. 4,000 in 512 53.3 -> 45.1, 4 of up to 9,000 21.1 ->
+//    15.4 (8 of exactly 8,192, one whole round of the int8 kernel's one-wave
+//    work-groups, 35.8 -> 37.6).  From 16 tiles a split the two are within 4%
+//    (20.5 / 19.9, 30.8 / 29.5) and the int8 kernel stays.
+//  * 9 to 16 (a few query rows of one sequence), up to two work-groups per
+//    CU: the rows kernels stage the split through LDS for up to four blocks.
+//    4 rows x 32 q / 8 kv heads, dim 128, 16,001 tokens in splits of 512 /
+//    1,024 18.2 -> 14.9 / 25.6 -> 19.2, 4,000 tokens in 256 14.8 -> 12.6; dim
+//    64, 16,001 tokens in 512 13.3 -> 10.0.
+// 17 to 32 head-rows are two blocks that each read the KV (19.6 against 22.8
+// at dim 128, 512-token splits) and stay on the rows kernels.
+bool one_block_rows(const SplitArgs& a) {
+  const uint64_t hr = uint64_t(a.rows) * a.group;
+  if (hr <= 4u || hr > 16u || (a.dim != 64 && a.dim != 128) || !generic_mfma_supported(a, true)) return false;
+  if (hr <= 8u) return a.split_tokens <= 15u * 64u;
+  return a.seq_starts == nullptr && uint64_t(a.splits) * a.kv_heads <= 512u;
+}
+
 hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t stream) {
   if (int8 && i8_wide_supported(a)) return launch_split_i8_wide(a, stream);
   if (generic_mfma_supported(a, int8)) {

@@ -427,7 +427,6 @@ hipError_t launch_dim(const SplitArgs& a, int cfg, hipStream_t stream) {
     return cfg == 42 ? launch_cfg<D, 4, 2, 4>(a, stream) : launch_cfg<D, 2, 2, 4>(a, stream);
   }
   if constexpr (D <= 128) {
-    if (cfg == 41) return launch_cfg<D, 4, 1, 8>(a, stream);
     if (cfg == 12) return launch_cfg<D, 1, 2, 8>(a, stream);
     return cfg == 42 ? launch_cfg<D, 4, 2, 8>(a, stream) : launch_cfg<D, 2, 2, 8>(a, stream);
   }
@@ -440,7 +439,6 @@ hipError_t preload_dim() {
   if constexpr (D <= 128) {
     e = preload_cfg<D, 8, 2, 4>();
     if (e == hipSuccess) e = preload_cfg<D, 8, 1, 4>();
-    if (e == hipSuccess) e = preload_cfg<D, 4, 1, 8>();
     if (e == hipSuccess) e = preload_cfg<D, 4, 2, 8>();
     if (e == hipSuccess) e = preload_cfg<D, 2, 2, 8>();
     if (e == hipSuccess) e = preload_cfg<D, 1, 2, 8>();

@@ -31,7 +31,6 @@ constexpr uint32_t kTiles = 64;  // tokens per tile
 //   8-tile splits   4,096 tokens 12.79 -> 12.04 (eight waves)
 //   16-tile splits  32,768 tokens 18.87 -> 18.38 (eight waves)
 //   32-tile splits  65,536 tokens 26.47 -> 27.80: chunks of four stay
-//   8 head-rows     4 tiles 18.32 -> 14.29, 8 tiles 18.50 -> 18.10, 16 tiles 20.37 -> 24.46
 //   dim 256         4 tiles 18.51 -> 15.21, 8 tiles 20.36 -> 19.63
 // Eight waves (two per SIMD, <= 256 registers each) where the state fits
 // (head_rows <= 4, dim <= 128) and the split has more than four tiles; else
@@ -63,7 +62,7 @@ int i8_config(const SplitArgs& a) {
   const uint32_t tiles = (a.split_tokens - 1u) / kTiles + 1u;
   const uint32_t hr = a.rows * a.group;
   const bool eight = hr <= 4 && a.dim <= 128;
-  if (forced == 42 || forced == 41 || forced == 22 || forced == 12 || ((forced == 82 || forced == 81) && eight))
+  if (forced == 42 || (forced == 41 && hr <= 4) || forced == 22 || forced == 12 || ((forced == 82 || forced == 81) && eight))
     return forced;
   const uint64_t groups = uint64_t(a.splits) * a.kv_heads * (a.seq_starts ? a.batch : 1u);
   if (groups > 512u) {
@@ -71,7 +70,7 @@ int i8_config(const SplitArgs& a) {
     return hr <= 4 ? 42 : 22;
   }
   if (eight) return tiles <= 4 ? 41 : (tiles < 16 ? 81 : 82);
-  return tiles <= 8 ? 41 : 42;
+  return hr <= 4 && tiles <= 8 ? 41 : 42;
 }
 
 }  // namespace

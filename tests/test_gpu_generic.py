@@ -29,6 +29,8 @@ SHAPES = [
     (1, 24, 4, 252, 16, 1100, 0, 1100, 1024, True, None),
     (1, 8, 2, 96, 16, 20000, 0, 20000, 20000, True, None),   # one split of 313 tiles: several row windows
     (3, 24, 8, 128, 64, 1500, 0, 1500, 256, True, [1499, 3, 700]),  # 9 head-rows of a tiled shape
+    (1, 10, 2, 64, 32, 3000, 0, 2990, 960, True, [2500]),    # 5 head-rows, fifteen tiles
+    (2, 16, 4, 128, 64, 1500, 33, 1500, 256, True, [1400, 900]),  # 8 head-rows in two rows
     (4, 16, 4, 64, 16, 1500, 5, 1490, 320, True, None),      # 16 head-rows, off-tile begin
     (2, 64, 8, 128, 32, 3000, 0, 3000, 1000, True, None),    # off-tile splits
     (1, 4, 4, 4, 16, 200, 0, 200, 64, False, None),
@@ -66,6 +68,7 @@ BATCHES = [
     (3, 24, 4, 256, 32, [200, 777], 128, True),         # 18 head-rows
     (1, 8, 2, 80, 16, [100, 4000, 33] * 20, 64, True),  # many work-groups
     (1, 8, 2, 64, 16, [300, 0, 17, 1000], 128, False),
+    (1, 64, 8, 128, 64, [300, 0, 17, 1000], 256, True),  # 8 head-rows of a tiled shape
 ]
 
 
