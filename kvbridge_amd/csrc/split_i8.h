@@ -47,6 +47,7 @@
 #include "batch.h"
 #include "device_common.h"
 #include "lds_stream.h"
+#include "split_generic.h"
 
 namespace kvb {
 namespace {

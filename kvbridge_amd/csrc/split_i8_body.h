@@ -6,7 +6,10 @@
 // digits of Q and of the weights:
 //  * ND = 3: Q as a 23-bit integer, weights below 2^21.
 //  * ND = 4: Q as a 31-bit integer (every bit of an fp32 Q within 2^-6 of the
-//    row's largest), weights below 2^28: as exact as fp32 arithmetic.
+//    row's largest), weights below 2^28: as exact as fp32 arithmetic.  Splits
+//    with values that such integers do not hold (NaN and infinities in Q, the
+//    scales or the scores; rows of Q or v-scales whose largest is below
+//    2^-70) go through the scalar rows of split_generic.h instead.
   SplitArgs a = a_in;
   a.begin = p_begin;
   a.end = p_end;
@@ -202,10 +205,17 @@
   // first KV item stays in flight) each wave reads its lanes' digits back.
   i32x4 qd[NCQ][KS];
   float cql[HS];
+  float odd = 0.f;  // four digits: NaN where a value needs the scalar rows
   static_assert(L::kQdBytes == NCQ * KS * 16, "digit bytes per lane");
   uint8_t* const qd_s = smem + L::kQd + lane * L::kQdBytes;
   {
     int kq_lane = 0;
+    if constexpr (ND == 4) {
+#pragma unroll
+      for (int nc = 0; nc < NCQ; ++nc)
+#pragma unroll
+        for (int i = 0; i < 16 * KS; ++i) odd = fmaf(qv[nc][i], 0.f, odd);
+    }
     auto col_kq = [&](float amax) __attribute__((always_inline)) {
       amax = rows_max(amax);
       int kq = 0;
@@ -213,6 +223,7 @@
         // |2^kq q| < 2^22 (three digits) or 2^30 (four): top digit in [-64, 64]
         kq = (ND == 3 ? 22 : 30) - __builtin_amdgcn_frexp_expf(amax);
         kq = kq < -100 ? -100 : (kq > 100 ? 100 : kq);
+        if constexpr (ND == 4) odd = amax < 0x1p-70f ? __builtin_nanf("") : odd;
       }
       return kq;
     };
@@ -363,7 +374,9 @@
     const float ks_l = __uint_as_float(it.ks);
     const float vs_l = __uint_as_float(it.vs);
     vsc[r] = vs_l;  // for the tile's V item (which loads no scales)
-    vmx = fmaxf(vmx, tok_ok ? fabsf(vs_l) : 0.f);
+    const float va = tok_ok ? fabsf(vs_l) : 0.f;
+    vmx = fmaxf(vmx, va);
+    if constexpr (ND == 4) odd = fmaf(va, 0.f, odd);
 #pragma unroll
     for (int h = 0; h < HS; ++h) {
       float si = fmaf(fmaf(float(dv[h][0]), 256.f, float(dv[h][1])), 256.f, float(dv[h][2]));
@@ -442,6 +455,7 @@
     if (vmax > 0.f) {
       kp = (ND == 3 ? 21 : 28) - __builtin_amdgcn_frexp_expf(vmax * kVmaxMargin);
       kp = kp < -100 ? -100 : (kp > 100 ? 100 : kp);
+      if constexpr (ND == 4) odd = vmax < 0x1p-70f || vmax > 0x1p126f ? __builtin_nanf("") : odd;
     }
 #pragma unroll
     for (int h = 0; h < HS; ++h) mu[h] = (m_new[h] == neg_inf() ? 0.f : m_new[h]) - (ND == 4 ? 0.f : float(kp));
@@ -533,6 +547,7 @@
 #pragma unroll
   for (int h = 0; h < HS; ++h) {
     const float lsum = wave_sum(lrun[h]);
+    if constexpr (ND == 4) odd = fmaf(lsum, 0.f, odd);
     if (lane == 0) {
       wm_s[wave * HS + h] = m_run[h] * kLn2;
       wl_s[wave * HS + h] = lsum;
@@ -549,7 +564,24 @@
       *reinterpret_cast<float4*>(&wacc_s[(wave * HS + n) * D + 16 * mb + 4 * g]) = y;
     }
   }
-  __syncthreads();
+  if constexpr (ND == 4) {
+    __shared__ uint32_t odd_s[NW];
+    const bool any = __ballot(odd != 0.f) != 0u;
+    if (lane == 0) odd_s[wave] = any ? 1u : 0u;
+    __syncthreads();
+    uint32_t rows_too = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) rows_too |= odd_s[w];
+    if (__builtin_amdgcn_readfirstlane(rows_too) != 0u) {
+      static_assert(sizeof(GenericLds<64 * NW>) <= size_t(L::kBytes), "the scalar rows fit the kernel's LDS");
+      auto& rows_lds = *reinterpret_cast<GenericLds<64 * NW>*>(smem);
+      for (uint32_t hh = 0; hh < head_rows; ++hh)
+        split_generic_row<true, 64 * NW>(a, (hh / a.group) * a.q_heads + kv * a.group + hh % a.group, split, rows_lds);
+      return;
+    }
+  } else {
+    __syncthreads();
+  }
   // One numerator column per thread and iteration (no branches: the LDS
   // loads of all waves are requested together); the thread of column 0 also
   // writes the head-row's maximum and denominator.

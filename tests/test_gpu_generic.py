@@ -198,3 +198,47 @@ def test_four_digit_batches(gpu, cfg):
         got = n.reshape(-1, 128)[sl].astype(np.float64) / l[sl, None].astype(np.float64)
         err = np.abs(got - ref.reshape(got.shape)).max(1) / np.abs(ref.reshape(got.shape)).max(1)
         assert g["strict_pass"] and err.max() <= 1e-6, (b, err.max())
+
+
+WIDE_ODD = NON_FINITE + ["q_inf", "v_scale_tiny", "q_tiny", "v_scale_huge"]
+
+
+@pytest.mark.parametrize("split", [128, 512, 1024])  # one, four and two or more tiles per wave
+@pytest.mark.parametrize("what", WIDE_ODD)
+def test_four_digit_batches_on_values_outside_fixed_point(gpu, what, split):
+    """Infinities, NaN and magnitudes that the digits cannot hold: as the
+    scalar kernel, which the same tokens in pages of 8 slots reach."""
+    bc = W.synth_batch(1, 8, 2, 128, 16, [400, 30], seed=9, split_tokens=split)
+    bc.qpos[0] = 370
+    tok = {"v_nan_masked": 380, "scale_inf_masked": 390}.get(what, 123)
+    pg, sl = int(bc.table[int(bc.page_offsets[0]) + tok // 16]), tok % 16
+    if what == "v_inf_zero_weight":
+        bc.vs[pg, 0, sl] = np.inf
+        bc.ks[pg, 0, sl] *= np.float32(1e6)
+    elif what in ("v_nan_masked", "scale_nan"):
+        bc.vs[pg, 0, sl] = np.nan
+    elif what in ("k_nan", "k_inf"):
+        bc.ks[pg, 0, sl] = np.nan if what == "k_nan" else np.inf
+    elif what in ("q_nan", "q_inf"):
+        bc.q[2 * 128 + 11] = np.nan if what == "q_nan" else np.inf
+    elif what == "scale_inf_masked":
+        bc.ks[pg, 0, sl], bc.vs[pg, 0, sl] = np.inf, np.nan
+    elif what == "v_scale_tiny":
+        bc.vs *= np.float32(2.0 ** -100)
+    elif what == "v_scale_huge":
+        bc.vs[pg, 0, sl] = np.float32(2.0 ** 126.5)
+    else:  # scores of ordinary size from tiny queries
+        bc.q *= np.float32(2.0 ** -100)
+        bc.ks *= np.float32(2.0 ** 100)
+    db = DeviceBatch(bc.shape, bc.to_device("cuda:0"))
+    assert ": split_i8_wide_kernel<128," in kvb.batch_kernel_name(bc.shape, db.inp)
+    other = _repage(bc.sequence(0), 8)
+    dc = DeviceCase(other)
+    assert ":" not in kvb.selected_kernel_name(other.shape, dc.inp, split)
+    got = [x[:size] for x, size in zip(db.run(fused=False)[:3], (8, 8, 8 * 128))]
+    for x, y, nm in zip(got, dc.run_decode(split)[0], "mln"):
+        assert np.array_equal(np.isnan(x), np.isnan(y)) and np.array_equal(np.isinf(x), np.isinf(y)), nm
+        fin = np.isfinite(y)
+        log(f"  {what} split={split} {nm}: {np.count_nonzero(~fin)} non-finite")
+        if fin.any():
+            np.testing.assert_allclose(x[fin], y[fin], rtol=5e-5, atol=3e-6 * np.abs(y[fin]).max())
