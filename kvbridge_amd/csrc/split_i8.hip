@@ -19,6 +19,16 @@ namespace {
 
 constexpr uint32_t kTiles = 64;  // tokens per tile
 
+// One head-row of one sequence, dim 128, splits of 13 tiles or more: four waves
+// that each hold one chunk of four tiles, and the single launch.  us per call,
+// 256 work-groups, 12 / 13 / 14 / 15 tiles: 15.2 / 15.3 / 15.5 / 15.9; eight
+// waves in chunks of one, two launches, 15.0 / - / 16.9 / 17.3, single launch
+// - / 16.1 / 16.6 / 17.2; eight waves in chunks of four - / 18.2 / 18.4 / 18.5.
+// 4 head-rows at 15 tiles are faster in chunks of one (18.1 against 18.9).
+bool one_row_long(const SplitArgs& a) {
+  return a.rows * a.group == 1u && a.dim == 128u && a.seq_starts == nullptr && a.split_tokens > 12u * kTiles;
+}
+
 // (waves, ring slots) per work-group as 10 * NW + NB; NB = 1: one-tile chunks.
 //
 // A grid of at most two work-groups per CU of a 256-CU device is bound by
@@ -69,6 +79,7 @@ int i8_config(const SplitArgs& a) {
     if (tiles <= 32u) return 12;
     return hr <= 4 ? 42 : 22;
   }
+  if (tiles < 16u && one_row_long(a)) return 42;
   if (eight) return tiles <= 4 ? 41 : (tiles < 16 ? 81 : 82);
   return hr <= 4 && tiles <= 8 ? 41 : 42;
 }
@@ -97,6 +108,7 @@ bool i8_supported(const SplitArgs& a) {
 //   64 work-groups, 4 x 64 outputs, 4 tiles  7.6 / 8.2;  256, 1 x 128  11.0 / 10.0
 //   64 work-groups, 4 x 128 outputs, 8 tiles 11.4 / 12.0;  4 tiles 10.5 / 9.8
 //   256 work-groups, 1 x 128, 16 tiles 17.5 / 18.4
+// One head-row has the shortest merge and keeps it from 13 tiles (one_row_long).
 // Grids of more than two work-groups per CU (batches) also run two launches:
 // every work-group's ticket and the merges then sit between rounds of split
 // work (16 ragged sequences: 116 us for two launches against 121-123 us).
@@ -107,7 +119,7 @@ bool i8_fusable(const SplitArgs& a) {
   const uint32_t nw = uint32_t(i8_config(a)) / 10u, hr = a.rows * a.group, outputs = hr * a.dim;
   if (nw < 4u || hr > nw || outputs > 64u * nw) return false;
   const uint32_t tiles = (a.split_tokens - 1u) / kTiles + 1u;
-  return tiles >= 16u || (groups <= 128u && (outputs <= 256u || tiles >= 8u));
+  return one_row_long(a) || tiles >= 16u || (groups <= 128u && (outputs <= 256u || tiles >= 8u));
 }
 
 hipError_t launch_i8_fenced_d128(const SplitArgs& a, hipStream_t stream);

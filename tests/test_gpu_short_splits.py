@@ -26,6 +26,7 @@ SHAPES = [
     (1, 8, 8, 128, 64, 9000, 0, 1024, None),   # sixteen: chunks of four tiles again
     (2, 8, 2, 128, 64, 1500, 0, 256, [1499, 20]),  # 8 head-rows, four waves
     (1, 16, 2, 64, 16, 2000, 0, 576, None),    # 8 head-rows, nine tiles
+    (1, 8, 8, 128, 64, 26600, 0, 832, None),   # thirteen tiles, 256 work-groups: single launch
     (1, 4, 4, 256, 64, 1200, 0, 256, None),    # dim 256, one head-row: single launch
     (1, 8, 2, 256, 32, 1200, 0, 512, None),    # dim 256, four head-rows: two launches
 ]
@@ -62,3 +63,5 @@ def test_single_launch_rule(gpu):
     assert fused(2, 4, 64, 8192, 256) and fused(8, 4, 128, 4096, 512) and fused(8, 4, 128, 65536, 2048)
     assert not fused(8, 4, 128, 2048, 256) and not fused(8, 1, 128, 8192, 256)  # too many outputs / work-groups
     assert not fused(2, 4, 64, 4096, 64) and not fused(2, 8, 64, 65536, 2048)   # 64 splits / 8 head-rows
+    # one head-row over 256 work-groups: from 13 tiles
+    assert fused(8, 1, 128, 26600, 832) and not fused(8, 1, 128, 24500, 768) and not fused(8, 4, 128, 26600, 832)
