@@ -77,11 +77,6 @@ const char* i8_rows_kernel_name(const SplitArgs& a);
 // f16-MFMA LDS kernel.  KVB_SPLIT_IMPL=f16 forces the f16 kernels
 // (comparisons).
 hipError_t launch_split_fast(const SplitArgs& a, hipStream_t stream);
-// The four-digit int8 kernel of ragged batches over small pages.
-bool i8_wide_supported(const SplitArgs& a);
-hipError_t launch_split_i8_wide(const SplitArgs& a, hipStream_t stream);
-const char* i8_wide_kernel_name(const SplitArgs& a);
-hipError_t preload_i8_wide();
 hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t stream);
 // Kernel instance a launch would run (diagnostics, profiles).
 const char* lds_kernel_name(const SplitArgs& a);

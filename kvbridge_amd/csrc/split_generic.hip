@@ -3,8 +3,7 @@
 // pages or with many head-rows.  The MFMA kernels (split_generic_mfma.h) serve
 // the shapes they can load in whole 16-byte pieces, the scalar kernel here
 // (split_generic.h) the rest: dims that are not a multiple of 4, pages that
-// are not a multiple of 16 tokens.  Dim 128 batches over small pages with few
-// head-rows run the four-digit int8 kernel (split_i8_wide.hip).
+// are not a multiple of 16 tokens.
 //
 // Scalar kernel: grid x = row * q_heads + head, y = split, z = sequence of a
 // batched call; block of 256 threads (4 waves).
@@ -90,7 +89,6 @@ bool one_block_rows(const SplitArgs& a) {
 }
 
 hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t stream) {
-  if (int8 && i8_wide_supported(a)) return launch_split_i8_wide(a, stream);
   if (generic_mfma_supported(a, int8)) {
     const int nw = mfma_waves(a, int8);
     return int8 ? launch_generic_i8(a, nw, stream) : launch_generic_f32(a, nw, stream);
@@ -114,9 +112,7 @@ const char* generic_kernel_name(const SplitArgs& a, bool int8) {
   const char* const t = int8 ? "true" : "false";
   const char* const v = a.seq_starts != nullptr ? "true" : "false";
   const int at = std::snprintf(buf, sizeof(buf), "split_generic_kernel<%s, %s>", t, v);
-  if (int8 && i8_wide_supported(a))
-    std::snprintf(buf + at, sizeof(buf) - at, ": %s", i8_wide_kernel_name(a));
-  else if (generic_mfma_supported(a, int8))
+  if (generic_mfma_supported(a, int8))
     std::snprintf(buf + at, sizeof(buf) - at, ": split_generic_%s_kernel<%d, %d, %s>", int8 ? "i8" : "f32",
                   a.dim <= 64 ? 64 : (a.dim <= 128 ? 128 : 256), mfma_waves(a, int8), v);
   return buf;
@@ -132,9 +128,8 @@ hipError_t preload_generic() {
     const hipError_t e = hipFuncGetAttributes(&attr, f);
     if (e != hipSuccess) return e;
   }
-  hipError_t e = preload_generic_i8();
-  if (e == hipSuccess) e = preload_generic_f32();
-  return e == hipSuccess ? preload_i8_wide() : e;
+  const hipError_t e = preload_generic_i8();
+  return e != hipSuccess ? e : preload_generic_f32();
 }
 
 }  // namespace kvb

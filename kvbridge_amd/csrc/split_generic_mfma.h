@@ -26,7 +26,7 @@
 // work-group per head-row (32 q / 8 kv heads): dim 96, 8,000 tokens 132 ->
 // 13.2 us; fp32 KV, dim 128, 8,192 tokens 150 -> 25.6 us (16-token tiles on
 // 128 work-groups, 26 GB/s per CU); 32 sequences of 100 .. 4,000 tokens over
-// 16-token pages, dim 128, 916 -> 49 us.  Error against 64 bits: no larger
+// 16-token pages, dim 128, 915 -> 42.7 us.  Error against 64 bits: no larger
 // (n 4.9e-7 / 2.8e-7 / 3.0e-7 relative, 6.9e-7 / 3.6e-7 / 3.9e-7 scalar).
 //
 // Non-finite values: a masked token's K, V and scales never reach the

@@ -47,7 +47,6 @@
 #include "batch.h"
 #include "device_common.h"
 #include "lds_stream.h"
-#include "split_generic.h"
 
 namespace kvb {
 namespace {
@@ -196,9 +195,9 @@ __device__ __forceinline__ void issue_item(const IssueCtx& c, uint32_t tile, boo
   }
 }
 
-template <int D, int NW, int HS, int ND>
+template <int D, int NW, int HS>
 struct I8Layout {
-  static constexpr int NC = (ND * HS + 15) / 16;      // MFMA column tiles
+  static constexpr int NC = (3 * HS + 15) / 16;       // MFMA column tiles
   static constexpr uint32_t kExchCol = 272;           // int32 column of 64 tokens + pad
   static constexpr uint32_t kDigCol = 80;             // int8 column of 64 tokens + pad
   static constexpr uint32_t kExch = NC * 16 * kExchCol;
@@ -349,7 +348,6 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
     uint32_t p_page_tokens, uint32_t p_kv_heads, uint32_t p_pages, SplitArgs a_in,
     const float* __restrict__ q_in, const int64_t* __restrict__ qpos_in, const int64_t* __restrict__ kpos_in,
     const int8_t* __restrict__ vdata, float* __restrict__ scratch_in) {
-  constexpr int ND = 3;
 #include "split_i8_body.h"
 }
 

@@ -1,15 +1,5 @@
-// Body of the integer-MFMA split kernels (split_i8.h), included in each kernel
-// function: as a function of its own that two kernels share it changed the
-// register allocation of the production instance (26.75 -> 26.89 us at 32 q /
-// 8 kv heads, dim 128, 65,536 tokens).  Uses the kernel's template parameters
-// D, NW, NB, PT, HS, FUSED, VARLEN, FENCE, its arguments, and ND, the int8
-// digits of Q and of the weights:
-//  * ND = 3: Q as a 23-bit integer, weights below 2^21.
-//  * ND = 4: Q as a 31-bit integer (every bit of an fp32 Q within 2^-6 of the
-//    row's largest), weights below 2^28: as exact as fp32 arithmetic.  Splits
-//    with values that such integers do not hold (NaN and infinities in Q, the
-//    scales or the scores; rows of Q or v-scales whose largest is below
-//    2^-70) go through the scalar rows of split_generic.h instead.
+// Body of the integer-MFMA split kernel (split_i8.h), included in the kernel
+// function.
   SplitArgs a = a_in;
   a.begin = p_begin;
   a.end = p_end;
@@ -30,7 +20,8 @@
   const uint32_t* __restrict__ table = VARLEN ? a.page_table : table_in;
   float* __restrict__ scratch = VARLEN ? a.scratch : scratch_in;
   constexpr int CH = NB == 1 ? 1 : 4;  // tiles per two-pass chunk
-  using L = I8Layout<D, NW, HS, ND>;
+  using L = I8Layout<D, NW, HS>;
+  constexpr int ND = 3;  // int8 digits of Q and of the weights
   constexpr int NC = L::NC;  // MFMA column tiles of the digit columns (PV; QK unless PAIR)
   // Paired-row QK (dim 128, <= 4 head-rows): MFMA row m of M-block mb is
   // half m%2 (dims 64*(m%2) ..) of token 8*mb + m/2; column tile h of the Q
@@ -205,25 +196,16 @@
   // first KV item stays in flight) each wave reads its lanes' digits back.
   i32x4 qd[NCQ][KS];
   float cql[HS];
-  float odd = 0.f;  // four digits: NaN where a value needs the scalar rows
   static_assert(L::kQdBytes == NCQ * KS * 16, "digit bytes per lane");
   uint8_t* const qd_s = smem + L::kQd + lane * L::kQdBytes;
   {
     int kq_lane = 0;
-    if constexpr (ND == 4) {
-#pragma unroll
-      for (int nc = 0; nc < NCQ; ++nc)
-#pragma unroll
-        for (int i = 0; i < 16 * KS; ++i) odd = fmaf(qv[nc][i], 0.f, odd);
-    }
     auto col_kq = [&](float amax) __attribute__((always_inline)) {
       amax = rows_max(amax);
       int kq = 0;
       if (amax > 0.f) {
-        // |2^kq q| < 2^22 (three digits) or 2^30 (four): top digit in [-64, 64]
-        kq = (ND == 3 ? 22 : 30) - __builtin_amdgcn_frexp_expf(amax);
+        kq = 22 - __builtin_amdgcn_frexp_expf(amax);  // |2^kq q| < 2^22: top digit in [-64, 64]
         kq = kq < -100 ? -100 : (kq > 100 ? 100 : kq);
-        if constexpr (ND == 4) odd = amax < 0x1p-70f ? __builtin_nanf("") : odd;
       }
       return kq;
     };
@@ -374,13 +356,10 @@
     const float ks_l = __uint_as_float(it.ks);
     const float vs_l = __uint_as_float(it.vs);
     vsc[r] = vs_l;  // for the tile's V item (which loads no scales)
-    const float va = tok_ok ? fabsf(vs_l) : 0.f;
-    vmx = fmaxf(vmx, va);
-    if constexpr (ND == 4) odd = fmaf(va, 0.f, odd);
+    vmx = fmaxf(vmx, tok_ok ? fabsf(vs_l) : 0.f);
 #pragma unroll
     for (int h = 0; h < HS; ++h) {
-      float si = fmaf(fmaf(float(dv[h][0]), 256.f, float(dv[h][1])), 256.f, float(dv[h][2]));
-      if constexpr (ND == 4) si = fmaf(si, 256.f, float(dv[h][3]));
+      const float si = fmaf(fmaf(float(dv[h][0]), 256.f, float(dv[h][1])), 256.f, float(dv[h][2]));
       float s2 = si * (ks_l * cql[h]);
       if (!full && !(real && tok >= s0 && tok < eh[h])) s2 = neg_inf();
       if (uint32_t(h) >= head_rows) s2 = neg_inf();
@@ -396,22 +375,11 @@
     const uint32_t tok = t0 + lane;
     const bool real = i < nt;
     const bool tok_ok = real && ((t0 >= s0 && t0 + kTileTokens <= e_min) || (tok >= s0 && tok < e_max));
-    // Four digits: the weights stay in (0, 1] and 2^kp goes to the v-scale; in
-    // the exponent (three digits: mu below) it would cost their last bits.
-    const float vs_l = tok_ok ? (ND == 4 ? __builtin_amdgcn_ldexpf(vsc[r], kp) : vsc[r]) : 0.f;
+    const float vs_l = tok_ok ? vsc[r] : 0.f;
     static_for<0, HS>([&](auto hc) __attribute__((always_inline)) {
       constexpr uint32_t h = decltype(hc)::value;
-      const float w = __builtin_amdgcn_exp2f(sc[r][h] - mu[h]);  // w * 2^kp (four digits: w)
+      const float w = __builtin_amdgcn_exp2f(sc[r][h] - mu[h]);  // w * 2^kp
       lw[h] += w;
-      if constexpr (ND == 4) {
-        // p = w * v_scale truncated to an integer below 2^28: four 7-bit digits.
-        const uint32_t pi = uint32_t(int(w * vs_l));
-        dig_w[h * L::kDigCol] = uint8_t(pi >> 21);
-        dig_w[(HS + h) * L::kDigCol] = uint8_t((pi >> 14) & 0x7fu);
-        dig_w[(2 * HS + h) * L::kDigCol] = uint8_t((pi >> 7) & 0x7fu);
-        dig_w[(3 * HS + h) * L::kDigCol] = uint8_t(pi & 0x7fu);
-        return;
-      }
       // p = w * v_scale rounded to an integer (0 <= p < 2^21) in one fma:
       // 1.5 * 2^23 + p lies in [2^23, 2^24), where the float's ulp is 1, so
       // its low 22 bits are p mod 2^22 (two's complement), and bits 0-6,
@@ -453,12 +421,11 @@
     vmx = 0.f;
     kp = 0;
     if (vmax > 0.f) {
-      kp = (ND == 3 ? 21 : 28) - __builtin_amdgcn_frexp_expf(vmax * kVmaxMargin);
+      kp = 21 - __builtin_amdgcn_frexp_expf(vmax * kVmaxMargin);
       kp = kp < -100 ? -100 : (kp > 100 ? 100 : kp);
-      if constexpr (ND == 4) odd = vmax < 0x1p-70f || vmax > 0x1p126f ? __builtin_nanf("") : odd;
     }
 #pragma unroll
-    for (int h = 0; h < HS; ++h) mu[h] = (m_new[h] == neg_inf() ? 0.f : m_new[h]) - (ND == 4 ? 0.f : float(kp));
+    for (int h = 0; h < HS; ++h) mu[h] = (m_new[h] == neg_inf() ? 0.f : m_new[h]) - float(kp);
   };
 
   // ---- fold the chunk's int32 digit numerators into the fp32 state.
@@ -467,7 +434,7 @@
 #pragma unroll
     for (int h = 0; h < HS; ++h) {
       fh[h] = m_run[h] == neg_inf() ? 0.f : __builtin_amdgcn_exp2f(m_run[h] - m_new[h]);
-      lrun[h] = fmaf(lrun[h], fh[h], ND == 4 ? lw[h] : __builtin_amdgcn_ldexpf(lw[h], -kp));
+      lrun[h] = fmaf(lrun[h], fh[h], __builtin_amdgcn_ldexpf(lw[h], -kp));
       lw[h] = 0.f;
       m_run[h] = m_new[h];
     }
@@ -482,20 +449,15 @@
       for (int e = 0; e < 4; ++e) {
         // digit dg of head h is column dg*HS + h: tile (dg*HS+h)/16, lane shift (dg*HS)%16.
         const float x0 = float(acc_i[0][mb][e]);
-        float x1, x2, x3 = 0.f;
+        float x1, x2;
         if constexpr (HS <= 4) {
           x1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x0), 0x100 + HS, 0xF, 0xF, true));
           x2 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x0), 0x100 + 2 * HS, 0xF, 0xF, true));
-          if constexpr (ND == 4)
-            x3 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x0), 0x100 + 3 * HS, 0xF, 0xF, true));
         } else {
           x1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x0), 0x100 + (HS % 16), 0xF, 0xF, true));
           x2 = float(acc_i[NC - 1][mb][e]);  // column 2*HS + h = 16 + h for HS == 8
-          if constexpr (ND == 4)
-            x3 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x2), 0x100 + (HS % 16), 0xF, 0xF, true));
         }
-        float comb = fmaf(fmaf(x0, 128.f, x1), 128.f, x2);
-        if constexpr (ND == 4) comb = fmaf(comb, 128.f, x3);
+        const float comb = fmaf(fmaf(x0, 128.f, x1), 128.f, x2);
         acc_f[mb][e] = fmaf(acc_f[mb][e], f_lane, comb * inv);
       }
 #pragma unroll
@@ -547,7 +509,6 @@
 #pragma unroll
   for (int h = 0; h < HS; ++h) {
     const float lsum = wave_sum(lrun[h]);
-    if constexpr (ND == 4) odd = fmaf(lsum, 0.f, odd);
     if (lane == 0) {
       wm_s[wave * HS + h] = m_run[h] * kLn2;
       wl_s[wave * HS + h] = lsum;
@@ -564,24 +525,7 @@
       *reinterpret_cast<float4*>(&wacc_s[(wave * HS + n) * D + 16 * mb + 4 * g]) = y;
     }
   }
-  if constexpr (ND == 4) {
-    __shared__ uint32_t odd_s[NW];
-    const bool any = __ballot(odd != 0.f) != 0u;
-    if (lane == 0) odd_s[wave] = any ? 1u : 0u;
-    __syncthreads();
-    uint32_t rows_too = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) rows_too |= odd_s[w];
-    if (__builtin_amdgcn_readfirstlane(rows_too) != 0u) {
-      static_assert(sizeof(GenericLds<64 * NW>) <= size_t(L::kBytes), "the scalar rows fit the kernel's LDS");
-      auto& rows_lds = *reinterpret_cast<GenericLds<64 * NW>*>(smem);
-      for (uint32_t hh = 0; hh < head_rows; ++hh)
-        split_generic_row<true, 64 * NW>(a, (hh / a.group) * a.q_heads + kv * a.group + hh % a.group, split, rows_lds);
-      return;
-    }
-  } else {
-    __syncthreads();
-  }
+  __syncthreads();
   // One numerator column per thread and iteration (no branches: the LDS
   // loads of all waves are requested together); the thread of column 0 also
   // writes the head-row's maximum and denominator.

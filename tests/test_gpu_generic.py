@@ -167,8 +167,8 @@ def test_padded_merge(gpu, dim, tokens, rows):
     np.testing.assert_allclose(out.ravel(), (n.reshape(-1, dim) / l[:, None]).ravel(), rtol=1e-6)
 
 
-WIDE_BATCHES = [
-    # kv_heads, group, page, lengths, split: one per (waves, ring) choice
+SMALL_PAGE_BATCHES = [
+    # kv_heads, group, page, lengths, split
     (8, 4, 16, [300, 0, 1, 1000, 64, 777], 256),          # short splits, small grid
     (8, 4, 32, [5000, 1024, 2047], 1024),                 # 16 tiles
     (4, 3, 16, [130, 4000, 33, 0, 64] * 12, 256),         # four tiles, large grid
@@ -177,17 +177,17 @@ WIDE_BATCHES = [
 ]
 
 
-@pytest.mark.parametrize("cfg", WIDE_BATCHES)
-def test_four_digit_batches(gpu, cfg):
-    """The four-digit kernel is held to fp32 accuracy: error against FP64 at
-    most 1e-6 of each head-row's largest numerator (two fp32 roundings per
-    partial and merge step; weights rounded at 2^-28)."""
+@pytest.mark.parametrize("cfg", SMALL_PAGE_BATCHES)
+def test_small_page_batches(gpu, cfg):
+    """Batches over 16- and 32-token pages are held to fp32 accuracy: error
+    against FP64 at most 1e-6 of each head-row's largest numerator (two fp32
+    roundings per partial and merge step)."""
     kvh, group, p, lengths, st = cfg
     bc = W.synth_batch(1, kvh * group, kvh, 128, p, lengths, seed=kvh * group + p, split_tokens=st)
     db = DeviceBatch(bc.shape, bc.to_device("cuda:0"))
     name = kvb.batch_kernel_name(bc.shape, db.inp)
-    log(f"four-digit batch shape={bc.shape.as_tuple()} kernel={name}")
-    assert ": split_i8_wide_kernel<128," in name
+    log(f"small-page batch shape={bc.shape.as_tuple()} kernel={name}")
+    assert ": split_generic_i8_kernel<128," in name
     m, l, n, _ = db.run(fused=False)
     for b in range(min(6, len(lengths))):
         g = check_sequence_vs_oracle(bc, b, m, l, n, f"seq {b}")
@@ -200,14 +200,57 @@ def test_four_digit_batches(gpu, cfg):
         assert g["strict_pass"] and err.max() <= 1e-6, (b, err.max())
 
 
-WIDE_ODD = NON_FINITE + ["q_inf", "v_scale_tiny", "q_tiny", "v_scale_huge"]
+SPREADS = ["zero_weight", "plain_weight", "full_weight", "one_channel", "q_outlier"]
 
 
-@pytest.mark.parametrize("split", [128, 512, 1024])  # one, four and two or more tiles per wave
-@pytest.mark.parametrize("what", WIDE_ODD)
-def test_four_digit_batches_on_values_outside_fixed_point(gpu, what, split):
-    """Infinities, NaN and magnitudes that the digits cannot hold: as the
-    scalar kernel, which the same tokens in pages of 8 slots reach."""
+@pytest.mark.parametrize("ratio", [2.0 ** 7, 2.0 ** 12, 2.0 ** 20, 2.0 ** 30, 1e12])
+@pytest.mark.parametrize("page,split", [(16, 256), (32, 1024)])
+@pytest.mark.parametrize("what", SPREADS)
+def test_small_page_batches_over_wide_magnitudes(gpu, what, page, split, ratio):
+    """One visible token whose v-scale is `ratio` times the others' must not
+    take bits from them, whatever its weight (zero_weight: the weight
+    underflows; full_weight: it has nearly all of it) and also where its codes
+    are zero (one_channel: every channel but one, which is left out of the
+    comparison); nor may one element of Q that meets only zero codes.  Same
+    bound as test_small_page_batches: each weight and each element of Q keeps
+    its own 24 bits."""
+    bc = W.synth_batch(1, 8, 2, 128, page, [700, 30], seed=11, split_tokens=split)
+    pg, sl = int(bc.table[int(bc.page_offsets[0]) + 123 // page]), 123 % page
+    q = bc.q.reshape(-1, 8, 128)[0]
+    keep = np.ones(128, bool)
+    if what == "q_outlier":
+        bc.q.reshape(-1, 8, 128)[0, :, 5] = np.float32(ratio)
+        bc.k[..., 5] = 0
+    else:
+        bc.vs[pg, :, sl] *= np.float32(ratio)
+    if what in ("zero_weight", "full_weight"):  # along the mean query of the kv head's four head-rows, or against it
+        mean = q.reshape(2, 4, 128).mean(1)
+        code = np.rint(mean / np.abs(mean).max(1, keepdims=True) * 127).astype(np.int8)
+        bc.k[pg, :, sl] = -code if what == "zero_weight" else code
+        bc.ks[pg, :, sl] = np.float32(3.0 if what == "zero_weight" else 0.1)
+    elif what == "one_channel":
+        bc.v[pg, :, :, sl] = 0
+        bc.v[pg, :, 9, sl] = 127
+        keep[9] = False
+    db = DeviceBatch(bc.shape, bc.to_device("cuda:0"))
+    log(f"wide magnitudes {what} page={page} split={split} ratio={ratio:.1e} "
+        f"kernel={kvb.batch_kernel_name(bc.shape, db.inp)}")
+    m, l, n, _ = db.run(fused=False)
+    ref = O.fp64(bc.sequence(0), threads=8)[0].reshape(8, 128)[:, keep]
+    got = (n.reshape(-1, 128)[:8].astype(np.float64) / l[:8, None].astype(np.float64))[:, keep]
+    err = np.abs(got - ref).max(1) / np.abs(ref).max(1)
+    log(f"  largest error {err.max():.2e}")
+    assert err.max() <= 1e-6, err
+
+
+OUT_OF_RANGE = NON_FINITE + ["q_inf", "v_scale_tiny", "q_tiny", "v_scale_huge"]
+
+
+@pytest.mark.parametrize("split", [128, 512, 1024])  # one and two tiles per wave, and more
+@pytest.mark.parametrize("what", OUT_OF_RANGE)
+def test_small_page_batches_on_extreme_values(gpu, what, split):
+    """Infinities, NaN and extreme magnitudes: as the scalar kernel, which the
+    same tokens in pages of 8 slots reach."""
     bc = W.synth_batch(1, 8, 2, 128, 16, [400, 30], seed=9, split_tokens=split)
     bc.qpos[0] = 370
     tok = {"v_nan_masked": 380, "scale_inf_masked": 390}.get(what, 123)
@@ -231,7 +274,7 @@ def test_four_digit_batches_on_values_outside_fixed_point(gpu, what, split):
         bc.q *= np.float32(2.0 ** -100)
         bc.ks *= np.float32(2.0 ** 100)
     db = DeviceBatch(bc.shape, bc.to_device("cuda:0"))
-    assert ": split_i8_wide_kernel<128," in kvb.batch_kernel_name(bc.shape, db.inp)
+    assert ": split_generic_i8_kernel<128," in kvb.batch_kernel_name(bc.shape, db.inp)
     other = _repage(bc.sequence(0), 8)
     dc = DeviceCase(other)
     assert ":" not in kvb.selected_kernel_name(other.shape, dc.inp, split)
