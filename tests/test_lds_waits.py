@@ -5,6 +5,7 @@ vector-memory wait leaves no load of an older tile DMA group in flight
 (kvbridge_amd/csrc/check_vm_waits.py), with planted mistakes that each check
 must catch."""
 import os
+import re
 import subprocess
 import sys
 import tempfile
@@ -179,3 +180,21 @@ def test_hand_counted_vm_waits_hold_and_planted_short_tiles_are_caught(asm_files
         for name, (found, n, _) in planted.items():
             if n and ("split_i8_rows_pc_kernel" in name or "split_lds_kernel" in name):
                 assert found, f"{name}: planted short tiles not caught"
+
+
+def test_digit_prologue_of_the_int8_kernel_takes_two_selects(asm_files):
+    """One-wave instances, where every lane builds the digits of all its Q
+    elements before the work-group's first barrier: at most two selects an
+    element (three digits) at 4 head-rows, one at 8, whose column tiles hold
+    two digits and one; 80 more for validity, clamps and the rest."""
+    seen = 0
+    for dim, f in ((64, "split_i8_d64.s"), (128, "split_i8_d128.s")):
+        for m in re.finditer(r"^(\w*split_i8_kernelILi%dELi1E\w*):(.*?)^\.Lfunc_end" % dim, asm_files[f], re.M | re.S):
+            hs = 8 if "Li8E" in m.group(1) else 4
+            elements = 16 * (dim // 64) * (1 if hs == 4 and dim == 64 else 2)  # per lane, over its column tiles
+            if "Lb0ELb0ELb0EEEv" not in m.group(1):  # batched: the sequence search sits in front
+                continue
+            n = m.group(2).split("s_barrier")[0].count("v_cndmask")
+            assert n <= elements * (2 if hs == 4 else 1) + 80, (m.group(1), n)
+            seen += 1
+    assert seen == 8
