@@ -15,7 +15,13 @@
 //  * int8 KV (64-token tiles): the codes are converted to bf16 (exact, 8
 //    bits), Q and the weights are cut into three bf16 pieces (8 bits each:
 //    the 24 bits of an fp32 exactly), and v_mfma_f32_16x16x32_bf16 sums the
-//    exact products in fp32.
+//    exact products in fp32.  The maximum carries every rounding of its score
+//    into m and l, so a score takes as few as it can: Q comes times the score
+//    scale, the sums of the high pieces are kept from the low ones' bits, and
+//    one fma applies the k-scale.  Error of m against 64 bits, relative, dim
+//    256 / 128 / 64: 9.5e-8 / 6.5e-8 / 5.8e-8 with one sum and log2 units,
+//    5.2e-8 / 4.4e-8 / 3.9e-8 so; l 3.9e-7 / 2.5e-7 / 2.1e-7 -> 2.2e-7 /
+//    1.8e-7 / 1.4e-7.
 //  * fp32 KV (16-token tiles): v_mfma_f32_16x16x4_f32.
 //
 // What bounds it: below two work-groups per CU, latency -- the page table, Q
@@ -26,8 +32,8 @@
 // work-group per head-row (32 q / 8 kv heads): dim 96, 8,000 tokens 132 ->
 // 13.2 us; fp32 KV, dim 128, 8,192 tokens 150 -> 25.6 us (16-token tiles on
 // 128 work-groups, 26 GB/s per CU); 32 sequences of 100 .. 4,000 tokens over
-// 16-token pages, dim 128, 915 -> 42.7 us.  Error against 64 bits: no larger
-// (n 4.9e-7 / 2.8e-7 / 3.0e-7 relative, 6.9e-7 / 3.6e-7 / 3.9e-7 scalar).
+// 16-token pages, dim 128, 915 -> 42.0 us.  Error of n against 64 bits, relative:
+// 2.3e-7 / 4.4e-7 / 2.0e-7, scalar 4.0e-7 / 8.3e-7 / 3.9e-7.
 //
 // Non-finite values: a masked token's K, V and scales never reach the
 // arithmetic; a split whose result is not finite (infinities or NaN in the
@@ -187,23 +193,21 @@ union GenericSmem {
 
 // Combines the waves (the visible part of a short split: dim 128, 16
 // head-rows, 3.2 of the split kernel's 12.7 us while every thread computed the
-// factors and took one column per step; a quad per thread took 2 us off; m in
-// log2 units, l summed over the lanes of a head-row
-// already) and writes the block's partials; a block with a non-finite result
+// factors and took one column per step; a quad per thread took 2 us off; l
+// summed over the lanes of a head-row already) and writes the block's partials; a block with a non-finite result
 // goes through the scalar rows instead.
 template <int DP, int NW, bool kInt8>
 __device__ __forceinline__ void write_partials(const SplitArgs& a, const HeadLane& h, uint32_t kv, uint32_t hb,
-                                               uint32_t split, float m2, float l, const f32x4 (&acc)[DP / 16],
+                                               uint32_t split, float m, float l, const f32x4 (&acc)[DP / 16],
                                                GenericSmem<DP, NW>& sm) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 15u, g = lane >> 4;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t rows_here = h.hr - 16u * hb < 16u ? h.hr - 16u * hb : 16u;
-  constexpr float kLn2 = 0.6931471805599453f;
   __syncthreads();  // the main loop's area is free
   float z = l * 0.f;  // 0 while everything is finite, else NaN
   if (n < rows_here) {
     if (g == 0) {
-      sm.c.m[wave][n] = m2 * kLn2;
+      sm.c.m[wave][n] = m;
       sm.c.l[wave][n] = l;
     }
 #pragma unroll
@@ -284,7 +288,8 @@ struct OnlineState {
 #pragma unroll
     for (int mb = 0; mb < DP / 16; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  // y: the lane's scores in log2 units -> its weights.
+  // y: the lane's scores -> its weights.  Scores and maxima are in natural
+  // units: in log2 units the rounding of the constant would reach every weight.
   template <int N>
   __device__ __forceinline__ void weights(float (&y)[N]) {
     float t = y[0];
@@ -293,7 +298,7 @@ struct OnlineState {
     const float m_new = fmaxf(m, rows_max(t));
     const float mu = m_new == neg_inf() ? 0.f : m_new;
     if (__any(m_new > m)) {  // else every factor is 1
-      const float f = m == neg_inf() ? 0.f : __builtin_amdgcn_exp2f(m - mu);
+      const float f = m == neg_inf() ? 0.f : __builtin_amdgcn_exp2f((m - mu) * kLog2e);
       l *= f;
 #pragma unroll
       for (int mb = 0; mb < DP / 16; ++mb) acc[mb] *= f;
@@ -302,7 +307,7 @@ struct OnlineState {
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      y[i] = __builtin_amdgcn_exp2f(y[i] - mu);
+      y[i] = __builtin_amdgcn_exp2f((y[i] - mu) * kLog2e);
       s += y[i];
     }
     l += s;
@@ -360,7 +365,9 @@ void split_generic_i8_kernel(SplitArgs a) {
   RowWindow win{0u, 0u, 0u};
   PageWindow next_win = load_window<TILE>(a, s, 0u, lane);
   const int64_t klast = a.k_positions[s.s1 - 1u], qpos = a.q_positions[block_row(a, hb, lane)];
-  // Q of this lane's head-row: dims 64 s + 16 g .. + 15 of step s, as bf16 pieces.
+  // Q of this lane's head-row times the score scale (rounded once per element,
+  // which averages out, instead of once per score): dims 64 s + 16 g .. + 15 of
+  // step s, as bf16 pieces.
   const uint32_t hr = a.rows * a.group, mine = 16u * hb + n;
   const bool real_head = mine < hr;
   float qv[KS][16];
@@ -376,7 +383,7 @@ void split_generic_i8_kernel(SplitArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float x = src[(in ? d : 0u) + i];
-          qv[k][4 * j + i] = in ? x : 0.f;
+          qv[k][4 * j + i] = in ? x * a.scale : 0.f;
         }
       }
   }
@@ -440,35 +447,56 @@ void split_generic_i8_kernel(SplitArgs a) {
     }
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the tiles stay in flight
 
-  const float cs = a.scale * kLog2e;
   for (uint32_t i = 0; i < nt; ++i) {
     const uint32_t t0 = (s.first + i * s.step) * TILE;
+    // The two low pieces of Q and the high one in accumulators of their own
+    // (cl, c): the high products are short, so their sum hardly rounds.  Up to
+    // dim 128 the low pieces of all steps go first, while the codes of the next
+    // step are converted; above, the converted codes would not fit.
     f32x4 c[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    f32x4 cl[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    constexpr bool kLowFirst = DP <= 128, kOneSum = DP == 64;
+    bf16x8 kb[kLowFirst ? 2 * KS : 1][4];
 #pragma unroll
-    for (int k = 0; k < KS; ++k)
+    for (int k = 0; k < 2 * KS; ++k) {
+      auto& kbs = kb[kLowFirst ? k : 0];
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        bf16x8 kb[4];
+      for (int mb = 0; mb < 4; ++mb)
+        kbs[mb] = codes_bf16(it.k[mb * KS + k / 2][2 * (k % 2)], it.k[mb * KS + k / 2][2 * (k % 2) + 1]);
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) kb[mb] = codes_bf16(it.k[mb * KS + k][2 * hf], it.k[mb * KS + k][2 * hf + 1]);
+      for (int p = 2; p >= (kLowFirst ? 1 : 0); --p) {
+        const bf16x8 qb = __builtin_bit_cast(bf16x8, sm.q[k / 2][k % 2][p][lane]);
 #pragma unroll
-        for (int p = 2; p >= 0; --p) {
-          const bf16x8 qb = __builtin_bit_cast(bf16x8, sm.q[k][hf][p][lane]);
-#pragma unroll
-          for (int mb = 0; mb < 4; ++mb) c[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[mb], qb, c[mb], 0, 0, 0);
+        for (int mb = 0; mb < 4; ++mb) {
+          f32x4& x = p == 0 ? c[mb] : cl[mb];
+          x = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kbs[mb], qb, x, 0, 0, 0);
         }
-        __builtin_amdgcn_sched_barrier(0);  // one step's operands at a time
       }
-    // Lane = token: the scale with the score factor, 0 for a token no row sees.
+      __builtin_amdgcn_sched_barrier(0);  // one step's operands at a time
+    }
+    if constexpr (kLowFirst) {
+#pragma unroll
+      for (int k = 0; k < 2 * KS; ++k) {
+        const bf16x8 qb = __builtin_bit_cast(bf16x8, sm.q[k / 2][k % 2][0][lane]);
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) {
+          f32x4& x = kOneSum ? cl[mb] : c[mb];  // two steps round little either way
+          x = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[k][mb], qb, x, 0, 0, 0);
+        }
+      }
+    }
+    // Lane = token: its scales, 0 for a token no row sees.
     const uint32_t tok = t0 + lane;
     const bool seen = tok >= s.s0 && tok < h.e_max;
-    float ksl = seen ? __uint_as_float(it.ks) * cs : 0.f;
+    float ksl = seen ? __uint_as_float(it.ks) : 0.f;
     float vsl = seen ? __uint_as_float(it.vs) : 0.f;
     asm volatile("" : "+v"(ksl), "+v"(vsl));  // the scales' registers are free for the next tile
     if (i + 1u < nt) window(i + 1u);
     issue_k(i + 1u, it);
     float y[16];
-#define KVB_SCORE(j) y[j] = c[(j) / 4][(j) % 4] * row_bcast<j>(ksl);
+#define KVB_SCORE(j)                                        \
+  y[j] = cl[(j) / 4][(j) % 4] * row_bcast<j>(ksl);          \
+  if constexpr (!kOneSum) y[j] = fmaf(c[(j) / 4][(j) % 4], row_bcast<j>(ksl), y[j]);
     KVB_SCORE(0) KVB_SCORE(1) KVB_SCORE(2) KVB_SCORE(3) KVB_SCORE(4) KVB_SCORE(5) KVB_SCORE(6) KVB_SCORE(7)
     KVB_SCORE(8) KVB_SCORE(9) KVB_SCORE(10) KVB_SCORE(11) KVB_SCORE(12) KVB_SCORE(13) KVB_SCORE(14) KVB_SCORE(15)
 #undef KVB_SCORE
@@ -586,7 +614,7 @@ void split_generic_f32_kernel(SplitArgs a) {
   window(0u);
   issue_k(0u, it);
   issue_v(0u, it);
-  const float cs = a.scale * kLog2e;
+  const float cs = a.scale;
   const bool ragged_dim = a.dim < uint32_t(DP);
   for (uint32_t i = 0; i < nt; ++i) {
     const uint32_t t0 = (s.first + i * s.step) * TILE;

@@ -61,6 +61,36 @@ def test_generic_mfma_shapes(gpu, cfg):
         assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
 
 
+@pytest.mark.parametrize("dim", [64, 96, 128, 192, 252])
+def test_generic_int8_scores_round_little(gpu, dim):
+    """m and l of the int8 MFMA kernel against FP64.  One rounding to fp32 has
+    a relative rms of 2^-25 / sqrt(3) .. 2^-24 / sqrt(3), 2.4e-8 over the
+    mantissas.  A score takes the rounding of its product with the k-scale, of
+    Q times the scale (less: it averages out over the elements) and of the sums
+    of the high pieces (the products are short: at most three in effect), so m
+    is within 2.4e-8 * sqrt(6) = 6e-8; l = sum of e^(score - m) carries m's own
+    absolute error (m is about 4) to 2.4e-7."""
+    err = []
+    for seed in (1, 2, 3, 4):
+        case = W.synth_case(4, 32, 8, dim, 16, 4000, seed=seed)
+        s = case.shape
+        dc = DeviceCase(case)
+        assert "split_generic_i8_kernel" in kvb.selected_kernel_name(s, dc.inp, 256)
+        m, l, _ = dc.run_decode(256)[0]
+        tok = np.arange(s.tokens)
+        pg, sl = case.table[tok // 16].astype(np.int64), tok % 16
+        k = case.k[pg, :, sl].astype(np.float64) * case.ks[pg, :, sl].astype(np.float64)[..., None]  # [t, kv, dim]
+        q = case.q.reshape(4, 8, 4, dim).astype(np.float64)
+        score = np.einsum("rhgd,thd->rhgt", q, k) * np.float64(np.float32(s.scale))
+        score[np.broadcast_to((case.kpos[None, :] > case.qpos[:, None])[:, None, None, :], score.shape)] = -np.inf
+        top = score.max(-1)
+        ref = top.ravel(), np.exp(score - top[..., None]).sum(-1).ravel()
+        err.append([np.linalg.norm(x - r) / np.linalg.norm(r) for x, r in zip((m, l), ref)])
+    em, el = np.mean(err, axis=0)
+    log(f"  dim {dim}: m {em:.2e} l {el:.2e}")
+    assert em <= 6e-8 and el <= 2.4e-7
+
+
 BATCHES = [
     # rows, q_heads, kv_heads, dim, page, lengths, split, int8
     (1, 32, 8, 128, 48, [300, 0, 1, 1000, 64], 256, True),
