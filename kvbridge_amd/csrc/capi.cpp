@@ -64,25 +64,6 @@ int hip_status(hipError_t e, const char* op) {
   return KVB_ERUNTIME;
 }
 
-// The same tokens counted from `begin`: where it lies on a page boundary but
-// off the 64-token tile grid (pages of 16 or 32 tokens) and more than 8
-// head-rows share a kv head, the page table, the key positions and the range
-// start there instead, so that the rows kernels, which need splits that start
-// on a tile, take the call.  Used by the whole calls; kvb_split_attention
-// runs its arguments as they are.  Dense geometry (rows 8, group 6, dim 256,
-// 32-token pages) through launch_attention_mma from token 32: 57,338 tokens
-// 286.6 -> 68.5 us, 8,000 tokens 56.3 -> 19.6, 1,500 tokens 28.6 -> 17.1 (the
-// f16 kernel reads the KV again for each of the three head-row blocks).
-kvbridge::Shape from_begin(kvbridge::Shape s, kvbridge::DeviceInput& in) {
-  const uint64_t head_rows = uint64_t(s.rows) * (s.q_heads / s.kv_heads);
-  if (s.begin % 64u == 0 || s.begin % s.page_tokens != 0 || s.begin == s.end || head_rows <= 8u) return s;
-  in.k_positions += s.begin;
-  in.page_table += s.begin / s.page_tokens;
-  s.end -= s.begin;
-  s.begin = 0;
-  return s;
-}
-
 // Split partials for a validated shape with `splits` splits of split_tokens.
 int run_split(const kvbridge::Shape& s, const kvbridge::DeviceInput& in, unsigned split_tokens,
               unsigned splits, float* scratch, hipStream_t stream, const char* op) {
@@ -207,7 +188,7 @@ static bool force_f16() {
 }
 
 hipError_t launch_split_fast(const SplitArgs& a, hipStream_t stream) {
-  if (!force_f16() && one_block_rows(a)) return launch_split_generic(a, true, stream);
+  if (!force_f16() && (one_block_rows(a) || off_grid_rows(a))) return launch_split_generic(a, true, stream);
   if (!force_f16() && i8_supported(a)) return launch_split_i8(a, stream);
   if (!force_f16() && i8_rows_supported(a)) return launch_split_i8_rows(a, stream);
   return launch_split_lds(a, stream);
@@ -215,7 +196,7 @@ hipError_t launch_split_fast(const SplitArgs& a, hipStream_t stream) {
 
 const char* split_kernel_name(const SplitArgs& a, bool tiled, bool int8) {
   if (!tiled) return generic_kernel_name(a, int8);
-  if (!force_f16() && one_block_rows(a)) return generic_kernel_name(a, true);
+  if (!force_f16() && (one_block_rows(a) || off_grid_rows(a))) return generic_kernel_name(a, true);
   if (!force_f16() && i8_supported(a)) return i8_kernel_name(a);
   if (!force_f16() && i8_rows_supported(a)) return i8_rows_kernel_name(a);
   return lds_kernel_name(a);
@@ -317,7 +298,7 @@ int kvb_launch_attention(const kvb_shape* sp, const kvb_device_input* ip, float*
   return guarded([&]() -> int {
     if (!sp || !ip) return fail(KVB_EINVAL, "shape and input descriptors must be non-null");
     const kvbridge::Shape s = to_shape(*sp);
-    kvbridge::DeviceInput in = to_input(*ip);
+    const kvbridge::DeviceInput in = to_input(*ip);
     if (const char* e = outputs_error(s, scratch, m, l, n)) return fail(KVB_EINVAL, e);
     if (const char* e = launch_error(s, in, scratch)) return fail(KVB_EINVAL, e);
     const unsigned splits = kvbridge::split_count(s);
@@ -326,7 +307,7 @@ int kvb_launch_attention(const kvb_shape* sp, const kvb_device_input* ip, float*
     // (src/attention_shared.cu:354-365): its shared-group kernel serves
     // group <= 8, its legacy per-head kernel larger groups.
     const bool legacy = s.q_heads / s.kv_heads > 8u;
-    int rc = run_split(from_begin(s, in), in, kvbridge::kSplitTokens, splits, scratch, st,
+    int rc = run_split(s, in, kvbridge::kSplitTokens, splits, scratch, st,
                        legacy ? "reference legacy split launch" : "reference split launch");
     if (rc != KVB_OK) return rc;
     return run_merge(s, scratch, splits, m, l, n, nullptr, KVB_OUT_NONE, st, "reference merge launch");
@@ -338,7 +319,7 @@ int kvb_launch_attention_mma(const kvb_shape* sp, const kvb_device_input* ip, fl
   return guarded([&]() -> int {
     if (!sp || !ip) return fail(KVB_EINVAL, "shape and input descriptors must be non-null");
     const kvbridge::Shape s = to_shape(*sp);
-    kvbridge::DeviceInput in = to_input(*ip);
+    const kvbridge::DeviceInput in = to_input(*ip);
     if (const char* e = outputs_error(s, scratch, m, l, n)) return fail(KVB_EINVAL, e);
     if (const char* e = launch_error(s, in, scratch)) return fail(KVB_EINVAL, e);
     if (!kvbridge::attention_mma_supported(s))
@@ -352,7 +333,7 @@ int kvb_launch_attention_mma(const kvb_shape* sp, const kvb_device_input* ip, fl
     // are 4- but not 16-byte aligned take the generic kernel (same results).
     const unsigned splits = kvbridge::split_count(s);
     const auto st = static_cast<hipStream_t>(stream);
-    int rc = run_split(from_begin(s, in), in, kvbridge::kSplitTokens, splits, scratch, st, "MMA split launch");
+    int rc = run_split(s, in, kvbridge::kSplitTokens, splits, scratch, st, "MMA split launch");
     if (rc != KVB_OK) return rc;
     return run_merge(s, scratch, splits, m, l, n, nullptr, KVB_OUT_NONE, st, "attention merge launch");
   });
@@ -421,7 +402,7 @@ int kvb_decode_attention(const kvb_shape* sp, const kvb_device_input* ip, uint32
   return guarded([&]() -> int {
     if (!sp || !ip) return fail(KVB_EINVAL, "shape and input descriptors must be non-null");
     const kvbridge::Shape s = to_shape(*sp);
-    kvbridge::DeviceInput in = to_input(*ip);
+    const kvbridge::DeviceInput in = to_input(*ip);
     if (const char* e = outputs_error(s, scratch, m, l, n)) return fail(KVB_EINVAL, e);
     if (const char* e = launch_error(s, in, scratch)) return fail(KVB_EINVAL, e);
     if (out_type != KVB_OUT_NONE && out_type != KVB_OUT_F32 && out_type != KVB_OUT_F16)
@@ -429,7 +410,7 @@ int kvb_decode_attention(const kvb_shape* sp, const kvb_device_input* ip, uint32
     if (out_type != KVB_OUT_NONE && !out) return fail(KVB_EINVAL, "output buffer must be non-null");
     const unsigned splits = kvbridge::split_count(s, split_tokens);
     const auto st = static_cast<hipStream_t>(stream);
-    int rc = run_split(from_begin(s, in), in, split_tokens, splits, scratch, st, "split launch");
+    int rc = run_split(s, in, split_tokens, splits, scratch, st, "split launch");
     if (rc != KVB_OK) return rc;
     return run_merge(s, scratch, splits, m, l, n, out, out_type, st, "attention merge launch");
   });

@@ -1,6 +1,7 @@
 // Split partials of every valid shape that the tiled kernels do not take:
-// fp32 KV, other dims, misaligned buffers, and ragged batches over small
-// pages or with many head-rows.  The MFMA kernels (split_generic_mfma.h) serve
+// fp32 KV, other dims, misaligned buffers, ragged batches over small pages or
+// with many head-rows, and the tiled shapes of one_block_rows and
+// off_grid_rows.  The MFMA kernels (split_generic_mfma.h) serve
 // the shapes they can load in whole 16-byte pieces, the scalar kernel here
 // (split_generic.h) the rest: dims that are not a multiple of 4, pages that
 // are not a multiple of 16 tokens.
@@ -86,6 +87,24 @@ bool one_block_rows(const SplitArgs& a) {
   if (hr <= 4u || hr > 16u || (a.dim != 64 && a.dim != 128) || !generic_mfma_supported(a, true)) return false;
   if (hr <= 8u) return a.split_tokens <= 15u * 64u;
   return a.seq_starts == nullptr && uint64_t(a.splits) * a.kv_heads <= 512u;
+}
+
+// More than 8 head-rows over a range that begins off the 64-token tile grid,
+// which the rows kernels do not take.  Like split_lds_kernel this one reads the
+// KV once per block of 16 head-rows, and it keeps 24 bits of a weight where
+// that one keeps 22 of f16 range: n is off by 3.1e-7 of 64 bits against 4e-6,
+// and a v-scale of 2^30 times the others' costs them nothing (3e-3 there).
+// us per call, split_lds_kernel -> this one, dense geometry (8 rows, group 6,
+// dim 256, 256-token splits) 1,500 / 8,000 / 57,338 tokens 28.7 -> 21.5 / 55.4
+// -> 41.2 / 286 -> 144; one 8,192-token split 276 -> 155; 8 rows x 32 q / 8 kv
+// heads, dim 128, 16,000 / 65,536 tokens 28.2 -> 23.7 / 74.3 -> 51.0; dim 64,
+// 65,536 tokens 72.7 -> 31.1; 512 head-rows 45.9 -> 39.9.  Counting the tokens
+// from the begin would let the rows kernels take page-aligned begins (57,338
+// tokens 55), but their weights are fixed point below the largest v-scale of
+// an epoch, where a v-scale of 2^20 times the others' leaves them an error of
+// 0.3 and a NaN becomes a number: not for calls that had neither.
+bool off_grid_rows(const SplitArgs& a) {
+  return uint64_t(a.rows) * a.group > 8u && a.begin % 64u != 0 && generic_mfma_supported(a, true);
 }
 
 hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t stream) {
