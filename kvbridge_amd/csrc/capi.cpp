@@ -64,12 +64,18 @@ int hip_status(hipError_t e, const char* op) {
   return KVB_ERUNTIME;
 }
 
+// Whether a call that splits and merges runs the generic kernels for its
+// splits.  kvb_split_attention alone keeps the f16 kernel off the tile grid.
+bool call_uses_generic(const kvbridge::Shape& s, const kvbridge::DeviceInput& in, const kvb::SplitArgs& a) {
+  return !kvb::tiled_supported(s, in) || (!kvb::force_f16() && kvb::off_grid_rows(a));
+}
+
 // Split partials for a validated shape with `splits` splits of split_tokens.
 int run_split(const kvbridge::Shape& s, const kvbridge::DeviceInput& in, unsigned split_tokens,
               unsigned splits, float* scratch, hipStream_t stream, const char* op) {
   const kvb::SplitArgs a = kvb::make_split_args(s, in, split_tokens, splits, scratch);
-  const hipError_t e = kvb::tiled_supported(s, in) ? kvb::launch_split_fast(a, stream)
-                                                   : kvb::launch_split_generic(a, s.int8, stream);
+  const hipError_t e = call_uses_generic(s, in, a) ? kvb::launch_split_generic(a, s.int8, stream)
+                                                   : kvb::launch_split_fast(a, stream);
   return hip_status(e, op);
 }
 
@@ -179,7 +185,7 @@ SplitArgs make_split_args(const kvbridge::Shape& s, const kvbridge::DeviceInput&
   return a;
 }
 
-static bool force_f16() {
+bool force_f16() {
   static const bool f = [] {
     const char* e = std::getenv("KVB_SPLIT_IMPL");
     return e && std::string(e) == "f16";
@@ -188,7 +194,7 @@ static bool force_f16() {
 }
 
 hipError_t launch_split_fast(const SplitArgs& a, hipStream_t stream) {
-  if (!force_f16() && (one_block_rows(a) || off_grid_rows(a))) return launch_split_generic(a, true, stream);
+  if (!force_f16() && one_block_rows(a)) return launch_split_generic(a, true, stream);
   if (!force_f16() && i8_supported(a)) return launch_split_i8(a, stream);
   if (!force_f16() && i8_rows_supported(a)) return launch_split_i8_rows(a, stream);
   return launch_split_lds(a, stream);
@@ -196,7 +202,7 @@ hipError_t launch_split_fast(const SplitArgs& a, hipStream_t stream) {
 
 const char* split_kernel_name(const SplitArgs& a, bool tiled, bool int8) {
   if (!tiled) return generic_kernel_name(a, int8);
-  if (!force_f16() && (one_block_rows(a) || off_grid_rows(a))) return generic_kernel_name(a, true);
+  if (!force_f16() && one_block_rows(a)) return generic_kernel_name(a, true);
   if (!force_f16() && i8_supported(a)) return i8_kernel_name(a);
   if (!force_f16() && i8_rows_supported(a)) return i8_rows_kernel_name(a);
   return lds_kernel_name(a);
@@ -376,8 +382,11 @@ int kvb_split_attention(const kvb_shape* sp, const kvb_device_input* ip, uint32_
     const kvbridge::DeviceInput in = to_input(*ip);
     if (const char* e = launch_error(s, in, scratch)) return fail(KVB_EINVAL, e);
     const unsigned splits = kvbridge::split_count(s, split_tokens);
-    return run_split(s, in, split_tokens, splits, scratch, static_cast<hipStream_t>(stream),
-                     "split launch");
+    const kvb::SplitArgs a = kvb::make_split_args(s, in, split_tokens, splits, scratch);
+    const auto st = static_cast<hipStream_t>(stream);
+    return hip_status(kvb::tiled_supported(s, in) ? kvb::launch_split_fast(a, st)
+                                                  : kvb::launch_split_generic(a, s.int8, st),
+                      "split launch");
   });
 }
 
@@ -527,7 +536,8 @@ const char* kvb_selected_kernel_name(const kvb_shape* sp, const kvb_device_input
   kvb::SplitArgs a = kvb::make_split_args(s, in, split_tokens, splits, nullptr);
   static uint32_t dummy_counter;  // only its non-nullness is read
   if (fused && kvb::tiled_supported(s, in) && kvb::i8_fusable(a)) a.counters = &dummy_counter;
-  return kvb::split_kernel_name(a, kvb::tiled_supported(s, in), s.int8);
+  const bool generic = fused ? call_uses_generic(s, in, a) : !kvb::tiled_supported(s, in);
+  return kvb::split_kernel_name(a, !generic, s.int8);
 }
 
 const char* kvb_batch_shape_error(const kvb_batch_shape* s) {

@@ -72,10 +72,11 @@ hipError_t launch_split_i8_rows(const SplitArgs& a, hipStream_t stream);
 bool i8_rows_supported(const SplitArgs& a);  // dim 128/256, one sequence, splits of <= 8/4 whole tiles
 const char* i8_rows_kernel_name(const SplitArgs& a);
 // The MFMA split path used by the entry points: the int8-MFMA kernel where
-// i8_supported (the generic MFMA kernel instead where one_block_rows or
-// off_grid_rows), else the int8-MFMA rows kernel where i8_rows_supported, else
-// the f16-MFMA LDS kernel.  KVB_SPLIT_IMPL=f16 forces the f16 kernels
+// i8_supported (the generic MFMA kernel instead where one_block_rows), else
+// the int8-MFMA rows kernel where i8_rows_supported, else the
+// f16-MFMA LDS kernel.  KVB_SPLIT_IMPL=f16 forces the f16 kernels
 // (comparisons).
+bool force_f16();
 hipError_t launch_split_fast(const SplitArgs& a, hipStream_t stream);
 hipError_t launch_split_generic(const SplitArgs& a, bool int8, hipStream_t stream);
 // Kernel instance a launch would run (diagnostics, profiles).
@@ -83,7 +84,8 @@ const char* lds_kernel_name(const SplitArgs& a);
 const char* i8_kernel_name(const SplitArgs& a);
 // Tiled shapes that the generic MFMA kernel serves faster: one block of 5 to 16 head-rows.
 bool one_block_rows(const SplitArgs& a);
-bool off_grid_rows(const SplitArgs& a);  // likewise: more head-rows, a range that begins off the tile grid
+// Likewise for calls that split and merge: more than 8 head-rows, a range that begins off the tile grid.
+bool off_grid_rows(const SplitArgs& a);
 bool generic_mfma_supported(const SplitArgs& a, bool int8);  // shapes of the generic MFMA kernels
 const char* generic_kernel_name(const SplitArgs& a, bool int8);
 const char* split_kernel_name(const SplitArgs& a, bool tiled, bool int8);
