@@ -223,13 +223,19 @@ int kvb_append_kv(const kvb_append_shape* s, const kvb_append_io* io, void* stre
 int kvb_decode_attention_noalloc(const kvb_shape* s, const kvb_device_input* in, uint32_t split_tokens, float* m,
                                  float* l, float* n, void* out, int out_type, void* stream);
 
-/* Extension (diagnostic): which split kernel kvb_split_attention would run for
- * these arguments: KVB_KERNEL_TILED_MFMA or KVB_KERNEL_GENERIC; 0 if invalid. */
+/* Extension (diagnostic): the class of these arguments for the split kernels:
+ * KVB_KERNEL_TILED_MFMA where shape and alignment admit the tiled MFMA kernels
+ * (int8 KV, dim 64/128/256, pages of whole 16-token groups, 16-byte aligned Q,
+ * K and V), else KVB_KERNEL_GENERIC; 0 if invalid.  Some admitted calls run the
+ * generic MFMA kernel all the same (5 to 16 head-rows over short splits or
+ * small grids): kvb_selected_kernel_name tells the kernel itself. */
 int kvb_selected_kernel(const kvb_shape* s, const kvb_device_input* in, uint32_t split_tokens);
 /* Extension (diagnostic): name of the kernel instance kvb_split_attention
  * (fused = 0) or kvb_decode_attention_fused (fused != 0) would launch, as
- * rocprofv3 reports it, e.g. "split_i8_kernel<128,8,2,true,4,false,false,false>"; "" if
- * the arguments are invalid.  Points to thread-local or static storage. */
+ * rocprofv3 reports it, e.g. "split_i8_kernel<128,8,2,true,4,false,false,false>"
+ * (the generic family with its MFMA instance after a colon,
+ * "split_generic_kernel<true, false>: split_generic_i8_kernel<128, 4, false>");
+ * "" if the arguments are invalid.  Points to thread-local or static storage. */
 const char* kvb_selected_kernel_name(const kvb_shape* s, const kvb_device_input* in, uint32_t split_tokens,
                                      int fused);
 

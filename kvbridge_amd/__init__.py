@@ -202,6 +202,8 @@ def decode_attention_noalloc(s: Shape, inp: DeviceInput, split_tokens: int, m, l
 
 
 def selected_kernel(s: Shape, inp: DeviceInput, split_tokens: int) -> int:
+    """Whether the tiled kernels admit these arguments (kvb_selected_kernel);
+    selected_kernel_name tells the kernel that would run."""
     return load().kvb_selected_kernel(ctypes.byref(s), ctypes.byref(inp), split_tokens)
 
 

@@ -124,6 +124,41 @@ def test_tiled_shapes(gpu, cfg):
     check_against_oracle(case, mln2, "launch_attention", ref, strict=True)
 
 
+NAMED_SHAPES = [
+    # rows, q_heads, kv_heads, dim, P, tokens, begin, end, split_tokens, instance of kvb_split_attention
+    (2, 16, 4, 128, 32, 2500, 37, 2490, 1024, "split_i8_kernel<128,4,2,false,8,"),   # 8 head-rows, off-tile begin
+    (1, 64, 8, 128, 64, 9000, 0, 9000, 2048, "split_i8_kernel<128,4,2,true,8,"),     # wide GQA, page tiles
+    (1, 64, 8, 128, 64, 70000, 0, 70000, 1024, "split_i8_kernel<128,1,2,true,8,"),   # one-wave work-groups
+    (1, 8, 1, 64, 16, 2100, 5, 2100, 1088, "split_i8_kernel<64,4,2,false,8,"),
+    (1, 20, 1, 64, 48, 960, 0, 955, 320, "split_lds_rows_kernel<64,16,false>"),      # 20 head-rows
+    (2, 48, 4, 64, 32, 1500, 0, 1500, 448, "split_lds_rows_kernel<64,16,false>"),
+    (3, 24, 4, 256, 32, 777, 0, 700, 250, "split_lds_kernel<256,4,1,false>"),        # off-tile splits
+    (6, 16, 4, 128, 48, 900, 0, 900, 250, "split_lds_kernel<128,4,1,false>"),
+    (5, 16, 4, 128, 64, 700, 0, 690, 96, "split_lds_kernel<128,4,1,true>"),
+    (3, 24, 8, 128, 64, 1500, 0, 1500, 256, "split_generic_kernel<true, false>: split_generic_i8_kernel<128,"),
+]
+
+
+@pytest.mark.parametrize("cfg", NAMED_SHAPES)
+def test_named_kernels(gpu, cfg):
+    """Shapes that each pin one kernel: kvb_selected_kernel says TILED_MFMA for
+    every shape the tiled kernels admit, also where the dispatch prefers the
+    generic MFMA kernel, so the instance name is asserted."""
+    rows, qh, kvh, d, p, t, b, e, st, name = cfg
+    case = W.synth_case(rows, qh, kvh, d, p, t, seed=zlib.crc32(repr(cfg).encode()) & 0xFFFF, begin=b, end=e)
+    dc = DeviceCase(case)
+    assert kvb.selected_kernel(case.shape, dc.inp, st) == kvb.KVB_KERNEL_TILED_MFMA
+    assert kvb.selected_kernel_name(case.shape, dc.inp, st).startswith(name)
+    scratch = dc.scratch(st)
+    kvb.split_attention(case.shape, dc.inp, st, scratch)
+    kvb.merge_finalize(case.shape, scratch, kvb.split_count(case.shape, st), dc.m, dc.l, dc.n)
+    # The f16 kernels cut Q and the weights into two f16 pieces (22 bits): 2^-22
+    # of scores of up to about 10 and of every weight, so a relative L2 of 1e-5;
+    # the per-element gate holds for the others.
+    g = check_against_oracle(case, dc.read(), name, strict="lds" not in name)
+    assert g["rel_l2"] <= 1e-5, g
+
+
 I8_ROWS_SHAPES = [
     # rows, q_heads, kv_heads, dim, P, tokens, begin, end, split_tokens, query positions, outliers
     (8, 24, 4, 256, 32, 2048, 0, 2048, 256, "causal", 0.0),    # the dense rows-8 / group-6 geometry
