@@ -101,7 +101,9 @@ __device__ __forceinline__ void merge_rows(uint32_t dim, uint32_t R, uint32_t S,
       const float lj = pj[1];
       const float mx = passes > 1u ? ml[4 * h] : wave_max(in ? mj : neg_inf());
       const float f = in && lj > 0.f ? exp_e(mj - mx) : 0.f;
-      const float lsum = wave_sum(f * lj);
+      // A split without a positive l_j (NaN among them) has no part in L; at the
+      // unpadded dims 0 * NaN reaches it.
+      const float lsum = wave_sum(!PAD || (in && lj > 0.f) ? f * lj : 0.f);
       if (lane < L::kPS) fs[h * L::kPS + lane] = f;
       if (lane == 0) {
         ml[4 * h] = mx;

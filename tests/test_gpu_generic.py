@@ -197,6 +197,39 @@ def test_padded_merge(gpu, dim, tokens, rows):
     np.testing.assert_allclose(out.ravel(), (n.reshape(-1, dim) / l[:, None]).ravel(), rtol=1e-6)
 
 
+@pytest.mark.parametrize("splits", [3, 64, 65])
+@pytest.mark.parametrize("dim", [60, 96, 252])
+def test_merge_leaves_non_finite_splits_out(gpu, dim, splits):
+    """L and N are sums over the splits with l_j > 0: a split whose l is NaN
+    (NaN of Q or of a K scale) reaches neither them nor the output, at 64
+    splits or fewer (padded merge) as above (scalar merge)."""
+    import torch
+
+    rng = np.random.default_rng(dim + splits)
+    s = W.synth_case(1, 8, 2, dim, 16, 64 * splits, seed=1).shape
+    parts = rng.standard_normal((8, splits, dim + 2)).astype(np.float32)
+    parts[..., 1] = rng.uniform(1, 60, (8, splits))
+    parts[0, 0, 1:] = np.nan           # the split that lanes past the last one read
+    parts[1, splits - 1, 1:] = np.nan
+    parts[2, :, 1:] = np.nan           # no split is left
+    parts[3, 1, 0], parts[3, 1, 1:] = -np.inf, 0.0
+    parts[4, 1, 1] = np.inf
+    good = (parts[..., 1] > 0)
+    top = parts[..., 0].astype(np.float64).max(1)
+    f = np.where(good, np.exp(parts[..., 0].astype(np.float64) - top[:, None]), 0.0)
+    l_ref = np.where(good, f * parts[..., 1], 0.0).sum(1)
+    n_ref = np.where(good[..., None], f[..., None] * parts[..., 2:], 0.0).sum(1)
+    sc = torch.from_numpy(parts).cuda()
+    m, l, n, out = (torch.empty(k, device="cuda") for k in (8, 8, 8 * dim, 8 * dim))
+    kvb.merge_finalize(s, sc, splits, m, l, n, out, kvb.KVB_OUT_F32)
+    torch.cuda.synchronize()
+    assert np.array_equal(m.cpu().numpy(), top.astype(np.float32))
+    np.testing.assert_allclose(l.cpu().numpy(), l_ref, rtol=1e-5)
+    np.testing.assert_allclose(n.cpu().numpy().reshape(8, dim), n_ref, rtol=1e-5, atol=1e-5 * np.abs(n_ref).max())
+    o_ref = np.where(l_ref[:, None] > 0, n_ref / np.where(l_ref > 0, l_ref, 1.0)[:, None], 0.0)
+    np.testing.assert_allclose(out.cpu().numpy().reshape(8, dim), o_ref, rtol=1e-5, atol=1e-5 * np.abs(o_ref).max())
+
+
 SMALL_PAGE_BATCHES = [
     # kv_heads, group, page, lengths, split
     (8, 4, 16, [300, 0, 1, 1000, 64, 777], 256),          # short splits, small grid
