@@ -245,8 +245,9 @@ const char* kvb_selected_kernel_name(const kvb_shape* s, const kvb_device_input*
  * agent-scope atomic partial stores and loads, without the L2 write-back and
  * invalidate these fences add).  Same arguments and results, bitwise; only
  * the eight-wave dim-128 single launch (<= 4 head-rows per kv head, pages of
- * >= 64 tokens, splits of >= 16 tiles) has an instance, other calls return
- * KVB_EINVAL.  For measuring that ordering choice, not for production use. */
+ * >= 64 tokens, splits of >= 16 tiles) has an instance; its calls over 33 to
+ * 128 splits are two launches, as there, and other calls return KVB_EINVAL.
+ * For measuring that ordering choice, not for production use. */
 int kvb_decode_attention_fused_fenced(const kvb_shape* s, const kvb_device_input* in, uint32_t split_tokens,
                                       float* scratch, uint32_t* counters, float* m, float* l, float* n, void* out,
                                       int out_type, void* stream);

@@ -481,6 +481,12 @@ int kvb_decode_attention_fused_fenced(const kvb_shape* sp, const kvb_device_inpu
       return fail(KVB_EINVAL,
                   "the fenced diagnostic call covers only the eight-wave dim-128 single launch "
                   "(<= 4 head-rows per kv head, pages of >= 64 tokens, splits of >= 16 tiles)");
+    if (!kvb::i8_fusable(a)) {  // two launches, as kvb_decode_attention_fused
+      const auto st = static_cast<hipStream_t>(stream);
+      const int rc = run_split(s, in, split_tokens, splits, scratch, st, "split launch");
+      if (rc != KVB_OK) return rc;
+      return run_merge(s, scratch, splits, m, l, n, out, out_type, st, "attention merge launch");
+    }
     return hip_status(kvb::launch_split_i8_fenced(a, static_cast<hipStream_t>(stream)), "fenced decode launch");
   });
 }

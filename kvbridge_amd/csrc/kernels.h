@@ -63,7 +63,8 @@ hipError_t launch_split_i8(const SplitArgs& a, hipStream_t stream);   // registe
 bool i8_supported(const SplitArgs& a);  // head_rows <= 8 (<= 4 at dim 256), power-of-two pages
 bool i8_fusable(const SplitArgs& a);    // the int8 kernel can run the fused merge
 // Diagnostic: the fused launch with formal release / acquire fences around
-// the merge ticket (eight-wave dim-128 page-tile configuration only).
+// the merge ticket (eight-wave dim-128 page-tile configuration only; the launch
+// itself only where i8_fusable).
 bool i8_fenced_supported(const SplitArgs& a);
 hipError_t launch_split_i8_fenced(const SplitArgs& a, hipStream_t stream);
 // Int8-MFMA kernel for more than 8 head-rows over short tile-aligned splits

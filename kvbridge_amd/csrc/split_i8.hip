@@ -125,14 +125,16 @@ bool i8_fusable(const SplitArgs& a) {
 hipError_t launch_i8_fenced_d128(const SplitArgs& a, hipStream_t stream);
 
 // Diagnostic single launch with formal release / acquire fences: only the
-// eight-wave dim-128 page-tile configuration (cfg2's) has an instance.
+// eight-wave dim-128 page-tile configuration (cfg2's) has an instance.  Calls
+// of that configuration whose merge is a launch of its own (33 to 128 splits)
+// need no fence: the second launch sees what the first one wrote.
 bool i8_fenced_supported(const SplitArgs& a) {
-  return a.dim == 128 && a.seq_starts == nullptr && a.page_tokens >= kTiles && i8_supported(a) && i8_fusable(a) &&
-         i8_config(a) == 82;
+  return a.dim == 128 && a.seq_starts == nullptr && a.page_tokens >= kTiles && i8_supported(a) &&
+         i8_config(a) == 82 && (i8_fusable(a) || (a.splits <= 128u && uint64_t(a.splits) * a.kv_heads <= 512u));
 }
 
 hipError_t launch_split_i8_fenced(const SplitArgs& a, hipStream_t stream) {
-  return i8_fenced_supported(a) ? launch_i8_fenced_d128(a, stream) : hipErrorInvalidValue;
+  return i8_fenced_supported(a) && i8_fusable(a) ? launch_i8_fenced_d128(a, stream) : hipErrorInvalidValue;
 }
 
 hipError_t launch_split_i8(const SplitArgs& a, hipStream_t stream) {

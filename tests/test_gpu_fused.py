@@ -157,3 +157,31 @@ def test_fenced_diagnostic_matches_fused(gpu):
         kvb.decode_attention_fused_fenced(small.shape, dcs.inp, 128, dcs.scratch(128),
                                           torch.zeros(2, dtype=torch.int32, device=dcs.device),
                                           dcs.m, dcs.l, dcs.n, None, kvb.KVB_OUT_NONE)
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,splits,taken", [(16, 4, 33, True), (8, 8, 64, True), (8, 4, 128, True),
+                                                           (8, 2, 129, False), (8, 8, 65, False)])
+def test_fenced_diagnostic_takes_long_merges(gpu, q_heads, kv_heads, splits, taken):
+    # 33 to 128 splits in at most 512 work-groups: the fenced call is the split
+    # and merge launches that the default call is there, bitwise the same.
+    import torch
+
+    s, t = W.torch_cache(1, q_heads, kv_heads, 128, 64, 1024 * splits, seed=93)
+    inp = kvb.device_input(t["q"], t["qpos"], t["kpos"], t["table"], t["k"], t["v"], t["ks"], t["vs"])
+    counters = torch.zeros(kv_heads, dtype=torch.int32, device="cuda")
+    res = []
+    for fn in (kvb.decode_attention_fused, kvb.decode_attention_fused_fenced):
+        sc, m, l, n = (torch.full((k,), float("nan"), device="cuda")
+                       for k in (kvb.scratch_elements(s, 1024), q_heads, q_heads, q_heads * 128))
+        out = torch.full((q_heads * 128,), float("nan"), dtype=torch.float16, device="cuda")
+        if fn is kvb.decode_attention_fused_fenced and not taken:
+            with pytest.raises(kvb.KvbInvalidArgument, match="fenced diagnostic"):
+                fn(s, inp, 1024, sc, counters, m, l, n, out, kvb.KVB_OUT_F16)
+            return
+        fn(s, inp, 1024, sc, counters, m, l, n, out, kvb.KVB_OUT_F16)
+        torch.cuda.synchronize()
+        assert torch.count_nonzero(counters).item() == 0
+        res.append([x.cpu().numpy().view(np.uint8) for x in (m, l, n, out)])
+    assert np.isfinite(res[0][0].view(np.float32)).all()
+    for x, y, nm in zip(*res, ("m", "l", "n", "out")):
+        assert np.array_equal(x, y), f"fenced call: {nm} differs"
