@@ -1,0 +1,51 @@
+"""Which kernel instance serves a call, on both sides of the lines where the
+measured order of the candidates changes (the comments at the rules hold the
+times).  Names only: no GPU."""
+import pytest
+
+import kvbridge_amd as kvb
+
+FAKE = kvb.device_input(*([0x1000] * 8))
+
+
+def name(kv_heads, head_rows, dim, splits, tiles, fused=False, page=64):
+    tokens = splits * tiles * 64
+    s = kvb.make_shape(1, kv_heads * head_rows, kv_heads, dim, page, -(-tokens // page), tokens, 0, tokens, 0.1)
+    return kvb.selected_kernel_name(s, FAKE, tiles * 64, fused)
+
+
+def waves_chunk(*args):
+    """(waves, one-tile chunks, single launch) of an int8 split kernel."""
+    n = name(*args)
+    assert n.startswith("split_i8_kernel<"), n
+    f = n[len("split_i8_kernel<"):-1].split(",")
+    return int(f[1]), f[2] == "1", f[5] == "true"
+
+
+@pytest.mark.parametrize("head_rows", [1, 2, 4])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_waves_of_short_splits(dim, head_rows):
+    """Eight waves hold a tile each while a work-group has the CU to itself;
+    with two per CU, and past 8 tiles (12 at dim 64), four waves are faster."""
+    for tiles, one_per_cu, two_per_cu in [(4, (4, True), (4, True)), (5, (8, True), (4, True)), (8, (8, True), (4, True)),
+                                          (9, (8, True) if dim == 64 else (4, False), (4, False)),
+                                          (12, (8, True) if dim == 64 else (4, False), (4, False)),
+                                          (13, (4, False), (4, False)), (15, (4, False), (4, False)),
+                                          (16, (8, False), (8, False))]:
+        assert waves_chunk(8, head_rows, dim, 32, tiles)[:2] == one_per_cu, tiles
+        assert waves_chunk(8, head_rows, dim, 33, tiles)[:2] == two_per_cu, tiles
+        assert waves_chunk(8, head_rows, dim, 64, tiles)[:2] == two_per_cu, tiles
+
+
+def test_waves_of_the_single_launch():
+    """The in-kernel merge wants a thread per output: eight waves to 12 tiles."""
+    assert waves_chunk(8, 4, 128, 4, 12, True) == (8, True, True)
+    assert waves_chunk(8, 1, 128, 4, 12, True) == (8, True, True)
+    assert waves_chunk(8, 1, 128, 4, 13, True) == (4, False, True)
+    assert waves_chunk(8, 4, 128, 4, 13, True) == (4, False, False)
+    assert waves_chunk(8, 4, 128, 16, 12, True) == (4, False, False)  # 16 splits of four head-rows: two launches
+
+
+def test_waves_at_dim_256():
+    assert waves_chunk(8, 4, 256, 32, 3)[:2] == (4, True) and waves_chunk(8, 4, 256, 33, 3)[:2] == (2, False)
+    assert waves_chunk(8, 4, 256, 33, 8)[:2] == (4, True) and waves_chunk(8, 4, 256, 32, 9)[:2] == (4, False)
