@@ -246,6 +246,21 @@ struct PackedPartials {
   }
 };
 
+// One column of a row-head's results.
+template <int D>
+__device__ __forceinline__ void store_result(const SplitArgs& a, size_t rh, uint32_t d, float m, float l, float n) {
+  if (d == 0) {
+    a.m[rh] = m;
+    a.l[rh] = l;
+  }
+  a.n[rh * D + d] = n;
+  if (a.out_type != 0) {
+    const float o = l > 0.f ? n / l : 0.f;
+    if (a.out_type == 1) static_cast<float*>(a.out)[rh * D + d] = o;
+    else static_cast<_Float16*>(a.out)[rh * D + d] = (_Float16)o;
+  }
+}
+
 // Merge of all splits of one kv head's head-rows, by the last work-group,
 // with the reference merge semantics (src/attention_shared.cu:295-335):
 // M = max_j m_j; L = sum_{l_j > 0} e^{m_j - M} l_j; N[d] likewise (N in four
@@ -314,18 +329,7 @@ __device__ __forceinline__ void fused_merge(const SplitArgs& a, uint32_t kv, uin
 #pragma unroll
     for (uint32_t j = 0; j < kCh; ++j) s4[j & 3u] = fmaf(fv[j], j <= jmax ? pre[j] : 0.f, s4[j & 3u]);
   }
-  const float nacc = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-  const size_t rh = row_head(hh);
-  if (d == 0) {
-    a.m[rh] = mx;
-    a.l[rh] = lsum;
-  }
-  a.n[rh * D + d] = nacc;
-  if (a.out_type != 0) {
-    const float ov = lsum > 0.f ? nacc / lsum : 0.f;
-    if (a.out_type == 1) static_cast<float*>(a.out)[rh * D + d] = ov;
-    else static_cast<_Float16*>(a.out)[rh * D + d] = (_Float16)ov;
-  }
+  store_result<D>(a, row_head(hh), d, mx, lsum, (s4[0] + s4[1]) + (s4[2] + s4[3]));
 }
 
 // VARLEN: batched call, grid (kv heads, splits, sequences) in the order of
@@ -904,7 +908,10 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
     const uint32_t row2 = hh / a.group, head2 = kv * a.group + hh % a.group;
     const size_t rh = size_t(row2) * a.q_heads + head2;
     float* const dst = scratch + (rh * a.splits + split) * W;
-    if constexpr (FUSED) {  // agent-coherent, in the merge's packed layout
+    if (FUSED && nsplit == 1u) {  // the merge of one split is the split itself
+      const float f = lsum > 0.f ? 1.f : 0.f;
+      store_result<D>(a, rh, d, mm, f * lsum, fmaf(f, val, 0.f));
+    } else if constexpr (FUSED) {  // agent-coherent, in the merge's packed layout
       const PackedPartials<D> pp(scratch, a);
       __hip_atomic_store(pp.n(rh, a.splits, split) + d, val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (d == 0) {
@@ -923,6 +930,7 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
   // ---- fused merge: the last work-group to finish for this kv head merges
   // its splits (agent-scope release of every partial, then a ticket).
   if constexpr (FUSED) {
+    if (nsplit == 1u) return;
     __shared__ uint32_t last_s;
     // The partials were stored with agent-scope atomic stores (coherent
     // across XCDs, no L2 write-back needed) and are read back with

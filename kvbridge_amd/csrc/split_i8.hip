@@ -106,9 +106,11 @@ bool i8_supported(const SplitArgs& a) {
 // launches.  The merge is one work-group per kv head with a thread per output
 // and a wave per head-row, at most 32 splits (otherwise the stand-alone merge,
 // whose work-groups spread over every CU, is faster: 8 head-rows, 32 splits
-// 14.3 against 21.5 us per call, 64 splits 8.5 against 11.0).  Short splits
-// leave the tickets and the merge nothing to hide behind, so below 16 tiles
-// only small grids keep it (us per call, single launch against two):
+// 14.3 against 21.5 us per call, 64 splits 8.5 against 11.0).  A split that is
+// alone needs no merge and is one launch whatever its shape (dim 256, 4
+// head-rows, 32 sequences of 8 / 20 tiles 18.9 / 37.6 against 23.4 / 42.3).
+// Short splits leave the tickets and the merge nothing to hide behind, so below
+// 16 tiles only small grids keep it (us per call, single launch against two):
 //   64 work-groups, 4 x 64 outputs, 4 tiles  7.6 / 8.2;  256, 1 x 128  11.0 / 10.0
 //   128 work-groups of 16 splits, 4 x 128 outputs, 11 tiles  13.2 / 12.8;  of 4
 //   splits 13.3 / 13.4
@@ -124,7 +126,9 @@ bool i8_fusable(const SplitArgs& a) {
   const uint64_t groups = uint64_t(a.splits) * a.kv_heads * (a.seq_starts ? a.batch : 1u);
   if (groups > 512u || a.splits > 32u) return false;
   const uint32_t nw = uint32_t(i8_config(a, true)) / 10u, hr = a.rows * a.group, outputs = hr * a.dim;
-  if (nw < 4u || hr > nw || outputs > 64u * nw) return false;
+  if (nw < 4u || hr > 4u) return false;
+  if (a.splits == 1u) return true;
+  if (outputs > 64u * nw) return false;
   const uint32_t tiles = (a.split_tokens - 1u) / kTiles + 1u;
   const bool one_row = hr == 1u && a.dim == 128u && a.seq_starts == nullptr && tiles > 12u;
   return one_row || tiles >= 16u || (groups <= 128u && (outputs <= 256u || (tiles >= 8u && a.splits <= 8u)));

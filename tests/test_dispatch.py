@@ -49,3 +49,11 @@ def test_waves_of_the_single_launch():
 def test_waves_at_dim_256():
     assert waves_chunk(8, 4, 256, 32, 3)[:2] == (4, True) and waves_chunk(8, 4, 256, 33, 3)[:2] == (2, False)
     assert waves_chunk(8, 4, 256, 33, 8)[:2] == (4, True) and waves_chunk(8, 4, 256, 32, 9)[:2] == (4, False)
+
+
+def test_a_lone_split_is_one_launch():
+    """At dim 256 the in-kernel merge serves one head-row; a split without
+    others needs none."""
+    for head_rows in (1, 2, 4):
+        assert waves_chunk(8, head_rows, 256, 1, 20, True)[2]
+        assert waves_chunk(8, head_rows, 256, 2, 20, True)[2] == (head_rows == 1)

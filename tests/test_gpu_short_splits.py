@@ -12,6 +12,7 @@ from kvbridge_amd import workloads as W
 from oracle import oracle as O
 
 from helpers import DeviceCase, check_against_oracle, log
+from test_gpu_batched import DeviceBatch, check_sequence_vs_oracle
 from test_gpu_fused import run_fused
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +66,24 @@ def test_single_launch_rule(gpu):
     assert not fused(2, 4, 64, 4096, 64) and not fused(2, 8, 64, 65536, 2048)   # 64 splits / 8 head-rows
     # one head-row over 256 work-groups: from 13 tiles
     assert fused(8, 1, 128, 26600, 832) and not fused(8, 1, 128, 24500, 768) and not fused(8, 4, 128, 26600, 832)
+
+
+@pytest.mark.parametrize("head_rows", [1, 3, 4])
+@pytest.mark.parametrize("dim,split", [(64, 512), (128, 256), (128, 2048), (256, 320), (256, 1024)])
+def test_lone_splits(gpu, dim, split, head_rows):
+    """Sequences of at most one split are one launch at any dim and up to four
+    head-rows, without a ticket: against the two launches, an empty sequence
+    and a row that sees nothing among them, and against FP64."""
+    bc = W.synth_batch(1, 2 * head_rows, 2, dim, 64, [split, 0, 1, split - 37, 200], seed=dim + head_rows,
+                       split_tokens=split)
+    bc.qpos[4] = -1
+    db = DeviceBatch(bc.shape, bc.to_device("cuda:0"))
+    assert kvb.batch_kernel_name(bc.shape, db.inp, True).split(",")[5] == "true"
+    db.counters.fill_(0)
+    one, two = db.run(fused=True), db.run(fused=False)
+    for x, y, nm in zip(one, two, ("m", "l", "n", "out")):
+        np.testing.assert_allclose(x, y, rtol=2e-6, atol=2e-6 * max(1.0, np.abs(y[np.isfinite(y)]).max()), err_msg=nm)
+    for b in (0, 1, 2, 3):
+        check_sequence_vs_oracle(bc, b, *one[:3], f"seq {b}")
+    rows = slice(4 * 2 * head_rows, 5 * 2 * head_rows)
+    assert np.isneginf(one[0][rows]).all() and not one[1][rows].any() and not one[3][rows].any()
