@@ -72,9 +72,17 @@ bool generic_mfma_supported(const SplitArgs& a, bool int8) {
 //    splits of 256, 8,192 tokens 14.4 -> 11.3, 65,536 tokens 45.3 -> 40.9; of
 //    512, 16,384 tokens 18.3 -> 14.1; dim 64, 16 q / 2 kv heads 12.6 -> 9.9;
 //    32 sequences of 100 .. 4,000 in 512 53.3 -> 45.1, 4 of up to 9,000 21.1 ->
-//    15.4 (8 of exactly 8,192, one whole round of the int8 kernel's one-wave
-//    work-groups, 35.8 -> 37.6).  From 16 tiles a split the two are within 4%
-//    (20.5 / 19.9, 30.8 / 29.5) and the int8 kernel stays.
+//    15.4.  From 16 tiles a split the two are within 4% (20.5 / 19.9, 30.8 /
+//    29.5) and the int8 kernel stays.  Above 512 work-groups that one runs four
+//    one-wave work-groups per CU and this one two of four waves, so at dim 128
+//    grids that all but fill the int8 kernel's first round stay there: 640 / 768
+//    / 896 / 1,024 / 1,152 work-groups, 8 head-rows, 4 tiles 19.7 / 20.2 / 22.0 /
+//    23.3 / 35.6 -> 19.6 / 20.2 / 23.6 / 24.4 / 27.2, 12 tiles 34.2 / 36.2 / 41.1
+//    / 43.8 / 66.4 -> 33.9 / 35.7 / 43.8 / 45.1 / 55.4; later rounds are within
+//    4% of each other.  Of a batch this holds where its sequences are as long as
+//    the longest (40 of 768 in 256 22.4 -> 26.2, but 40 of 90 .. 1,480 in 960 37.7
+//    -> 29.0).  Dim 64 gains on either side (12 tiles, 640 / 1,024 work-groups
+//    25.4 / 26.9 -> 19.5 / 24.7).
 //  * 9 to 16 (a few query rows of one sequence), up to two work-groups per
 //    CU: the rows kernels stage the split through LDS for up to four blocks.
 //    4 rows x 32 q / 8 kv heads, dim 128, 16,001 tokens in splits of 512 /
@@ -85,8 +93,12 @@ bool generic_mfma_supported(const SplitArgs& a, bool int8) {
 bool one_block_rows(const SplitArgs& a) {
   const uint64_t hr = uint64_t(a.rows) * a.group;
   if (hr <= 4u || hr > 16u || (a.dim != 64 && a.dim != 128) || !generic_mfma_supported(a, true)) return false;
-  if (hr <= 8u) return a.split_tokens <= 15u * 64u;
-  return a.seq_starts == nullptr && uint64_t(a.splits) * a.kv_heads <= 512u;
+  if (hr > 8u) return a.seq_starts == nullptr && uint64_t(a.splits) * a.kv_heads <= 512u;
+  if (a.split_tokens > 15u * 64u) return false;
+  const bool batch = a.seq_starts != nullptr;
+  if (a.dim == 64 || (batch && uint64_t(a.total_tokens) * 10u < uint64_t(a.batch) * a.max_tokens * 9u)) return true;
+  const uint64_t groups = uint64_t(a.splits) * a.kv_heads * (batch ? a.batch : 1u);
+  return groups < 768u || groups > 1024u;
 }
 
 // More than 8 head-rows over a range that begins off the 64-token tile grid,

@@ -57,3 +57,27 @@ def test_a_lone_split_is_one_launch():
     for head_rows in (1, 2, 4):
         assert waves_chunk(8, head_rows, 256, 1, 20, True)[2]
         assert waves_chunk(8, head_rows, 256, 2, 20, True)[2] == (head_rows == 1)
+
+
+@pytest.mark.parametrize("head_rows", [5, 8])
+def test_wide_gqa_over_the_int8_kernels_round(head_rows):
+    """5 to 8 head-rows over splits of up to 15 tiles: the generic MFMA kernel,
+    but not where the grid all but fills the first round of the int8 kernel's
+    one-wave work-groups at dim 128."""
+    def generic(dim, groups, tiles):
+        return ": split_generic_i8_kernel<" in name(8, head_rows, dim, groups // 8, tiles)
+
+    for tiles in (4, 12, 15):
+        assert [g for g in (64, 512, 760, 768, 1024, 1032, 1536, 2048) if not generic(128, g, tiles)] == [768, 1024]
+        assert all(generic(64, g, tiles) for g in (64, 512, 776, 1024, 2048))
+    assert not generic(128, 64, 16) and not generic(64, 64, 16)
+
+
+def test_wide_gqa_batches():
+    """The same grid of a batch: full sequences only."""
+    def generic(batch, max_tokens, total):
+        s = kvb.make_batch_shape(batch, 1, 64, 8, 128, 64, 1 << 14, max_tokens, total, 1 << 14, 512, 0.1, True)
+        return ":" in kvb.batch_kernel_name(s, kvb.batch_input(*([0x1000] * 10)))
+
+    assert not generic(8, 8192, 8 * 8192) and generic(8, 8192, 8 * 7000)
+    assert generic(40, 8192, 40 * 8192) and generic(4, 8192, 4 * 8192)
