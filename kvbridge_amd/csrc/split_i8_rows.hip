@@ -1324,18 +1324,42 @@ bool pc_shape(const SplitArgs& a) {
   return a.dim == 256 && hblocks <= kPcBlocks;
 }
 
+// Time of a grid with spw consecutive splits per work-group, in tiles that a CU
+// takes one after the other (the LDS holds one work-group per CU); the ends of a
+// work-group take as long as four tiles, six at dim 128.  The last work-group of
+// a kv head is shorter, and a last round of no more work-groups than those (up
+// to one per XCD) begins when they end.  The pc kernel streams a quarter slower
+// where a work-group's pages do not fit its window of 64.
+uint64_t rounds_tiles(const SplitArgs& a, uint32_t spw, uint32_t cus) {
+  const uint64_t per_head = (a.splits + spw - 1u) / spw, groups = per_head * a.kv_heads;
+  const uint64_t full = uint64_t(spw) * a.split_tokens, last = uint64_t(a.end - a.begin) - (per_head - 1u) * full;
+  const uint64_t before = (groups - 1u) / cus, in_last = groups - before * cus;
+  uint64_t tokens = before * full + (in_last <= a.kv_heads && in_last <= 8u ? last : full);
+  if (pc_shape(a) && full > 64u * uint64_t(a.page_tokens)) tokens += tokens / 4u;
+  return tokens / kTileTokens + (a.dim == 256 ? 4u : 6u) * (before + 1u);
+}
+
+// Short splits: several consecutive splits per work-group, as many as make one
+// work-group per CU.  Rounded up, as a few over cost a second round: rounded
+// down, us per call -> up, dense geometry, 256-token splits, 20,000 / 33,000 /
+// 57,338 tokens 33.3 -> 28.5 / 47.1 -> 39.0 / 68.5 -> 52.4; 8 rows x 32 q / 8 kv
+// heads, dim 128, 32,000 tokens 46.4 -> 33.7.  Rounded down where that is the
+// shorter by rounds_tiles: 30 head-rows, 8 kv heads, dim 256, 33 splits of 1,024
+// of which the last has 102 / 512 tokens, 64-token pages 44.7 / 51.8 against
+// 55.1 / 55.3 rounded up, 16-token pages 45.1 / 52.7 against 66.1.  Over 750 grids
+// of 260 to 520 work-groups the choice is within 7% of the better one.
+uint32_t splits_per_group(const SplitArgs& a) {
+  const uint32_t cus = device_cus();
+  const uint64_t n = uint64_t(a.splits) * a.kv_heads;
+  if (n <= cus) return 1u;
+  const uint32_t down = uint32_t(n / cus), up = uint32_t((n + cus - 1u) / cus);
+  return rounds_tiles(a, down, cus) < rounds_tiles(a, up, cus) ? down : up;
+}
+
 template <int D>
 hipError_t launch_dim(const SplitArgs& a, hipStream_t stream) {
-  // Short splits: several consecutive splits per work-group, as many as make
-  // one work-group per CU (rounded up: the LDS holds one per CU, so a few over
-  // cost a second round), when a split is a whole number of phases.  Rounded
-  // down, us per call -> up: dense geometry, 256-token splits, 20,000 / 33,000
-  // / 57,338 tokens 33.3 -> 28.5 / 47.1 -> 39.0 / 68.5 -> 52.4; 8 rows x 32 q /
-  // 8 kv heads, dim 128, 32,000 tokens 46.4 -> 33.7.
   uint32_t spw = 1u;
-  if ((a.split_tokens / kTileTokens) % RowsGeo<D>::kCT == 0u) {
-    spw = uint32_t((uint64_t(a.splits) * a.kv_heads + device_cus() - 1u) / device_cus());
-  }
+  if ((a.split_tokens / kTileTokens) % RowsGeo<D>::kCT == 0u) spw = splits_per_group(a);
   const dim3 grid((a.splits + spw - 1u) / spw, a.kv_heads);
   const bool pt = a.page_tokens % kTileTokens == 0;
   if constexpr (D == 256) {

@@ -30,6 +30,9 @@ SHAPES = [
     (1, 8, 8, 128, 64, 26600, 0, 832, None),   # thirteen tiles, 256 work-groups: single launch
     (1, 4, 4, 256, 64, 1200, 0, 256, None),    # dim 256, one head-row: single launch
     (1, 8, 2, 256, 32, 1200, 0, 512, None),    # dim 256, four head-rows: two launches
+    (3, 32, 8, 256, 64, 4136, 0, 128, None),   # rows kernel: 264 work-groups, the last of a head short
+    (3, 32, 8, 256, 64, 4224, 0, 128, [4000, 9, 4223]),  # the same, all full: two splits per work-group
+    (8, 32, 8, 128, 64, 8500, 0, 256, None),   # dim 128, 272 work-groups
 ]
 
 
