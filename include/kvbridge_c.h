@@ -104,18 +104,20 @@ int kvb_decode_attention(const kvb_shape* s, const kvb_device_input* in, uint32_
                          void* stream);
 /* Extension (no counterpart in the reference library; for decode loops that
  * want one launch per call): kvb_decode_attention as a single kernel where
- * the int8-MFMA split kernel serves the shape and its in-kernel merge is
- * short (at most two 16-byte-load passes over the splits) -- the last
+ * the int8-MFMA split kernel serves the shape with at most 4 head-rows per kv
+ * head and its in-kernel merge is short (at most 32 splits, of 16 tiles of 64
+ * tokens or more except in small grids; one split always) -- the last
  * work-group to finish for each kv head merges that head's splits
  * (log-sum-exp) into m, l, n and out.  Otherwise it runs the two launches of
  * kvb_decode_attention.  `counters` holds kv_heads uint32 that must be zero
  * before the first call; every call leaves them zero (allocate and zero them
  * once, e.g. next to the scratch buffer).  Calls sharing `counters` must not
- * overlap in time (same rule as for scratch).  m, l, n, out equal those of
- * kvb_decode_attention up to fp32 summation order in the merge.  What the
- * single launch leaves in scratch is internal: where its merge takes the
- * short path (<= 32 splits) the partials are packed in a layout of their
- * own, not the rows kvb_split_attention writes. */
+ * overlap in time (same rule as for scratch).  m equals that of
+ * kvb_decode_attention, l, n and out up to fp32 rounding (order of the sums in
+ * the merge and, for some split lengths, over the waves).  What the single
+ * launch leaves in scratch is internal: the partials are packed in a layout of
+ * their own, not the rows kvb_split_attention writes, and a split without
+ * others writes none. */
 int kvb_decode_attention_fused(const kvb_shape* s, const kvb_device_input* in, uint32_t split_tokens,
                                float* scratch, uint32_t* counters, float* m, float* l, float* n, void* out,
                                int out_type, void* stream);
@@ -165,9 +167,9 @@ int kvb_batch_output_scalar_elements(const kvb_batch_shape* s, size_t* elements)
  * int8-MFMA kernel serves the shape and its in-kernel merge is short (as
  * for kvb_decode_attention_fused), the last work-group of each
  * (sequence, kv head) merging its splits; otherwise two launches.  The
- * single launch writes partials only for each sequence's own splits (the
- * rest of that sequence's scratch block is left as it was), in the internal
- * layout of kvb_decode_attention_fused. */
+ * single launch writes partials only for each sequence's own splits, if there
+ * are several (the rest of that sequence's scratch block is left as it was), in
+ * the internal layout of kvb_decode_attention_fused. */
 int kvb_decode_attention_batched(const kvb_batch_shape* s, const kvb_batch_input* in, float* scratch,
                                  uint32_t* counters, float* m, float* l, float* n, void* out, int out_type,
                                  void* stream);

@@ -66,7 +66,10 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
 // sequences per round (a.packed: at most 256 sequences; above that the rounds
 // would cost more than the imbalance).  A grid of at most one work-group per
 // CU has nothing to balance and takes the block index as it is (two
-// sequences, 144 work-groups: 16.5 against 16.9 us).  Consecutive work-groups
+// sequences, 144 work-groups: 16.5 against 16.9 us).  Above that sequences of
+// one length pay 0.4 to 1.0 us for nothing (11 of 3,326 tokens, dim 64: 20.7 ->
+// 21.4), but the host sees neither lengths nor whether the declared totals are
+// capacities.  Consecutive work-groups
 // are the kv heads of one item, so each XCD gets the same share of every
 // sequence when there are 8 of them.
 __device__ __forceinline__ BatchItem batch_item(const SplitArgs& a) {

@@ -33,9 +33,10 @@ struct SplitArgs {
   float* n;
   void* out;
   int out_type;
-  // Batched call (kvb_decode_attention_batched): non-null seq_starts makes
-  // grid.z the sequence index b, and every work-group first rebases these
-  // arguments on sequence b (rebase_sequence, batch.h).  q, q_positions and
+  // Batched call (kvb_decode_attention_batched): with non-null seq_starts every
+  // work-group takes a (sequence b, split) -- the block index itself, or by
+  // live splits first where packed (batch_item, batch.h; the scalar kernel:
+  // grid.z) -- and rebases these arguments on b (rebase_sequence).  q, q_positions and
   // the outputs then hold `batch` consecutive blocks of rows * q_heads
   // row-heads, k_positions and page_table are concatenations indexed through
   // seq_starts / page_offsets, and `splits` is the partial stride of every
@@ -61,7 +62,7 @@ bool tiled_supported(const kvbridge::Shape& s, const kvbridge::DeviceInput& in);
 hipError_t launch_split_lds(const SplitArgs& a, hipStream_t stream);  // LDS-DMA-staged tiles, f16 MFMA
 hipError_t launch_split_i8(const SplitArgs& a, hipStream_t stream);   // register-staged tiles, int8 MFMA
 bool i8_supported(const SplitArgs& a);  // head_rows <= 8 (<= 4 at dim 256), power-of-two pages
-bool i8_fusable(const SplitArgs& a);    // the int8 kernel can run the fused merge
+bool i8_fusable(const SplitArgs& a);    // the call runs faster as one launch (fused merge)
 // Diagnostic: the fused launch with formal release / acquire fences around
 // the merge ticket (eight-wave dim-128 page-tile configuration only; the launch
 // itself only where i8_fusable).
@@ -70,7 +71,7 @@ hipError_t launch_split_i8_fenced(const SplitArgs& a, hipStream_t stream);
 // Int8-MFMA kernel for more than 8 head-rows over short tile-aligned splits
 // (one work-group per split and kv head, the split's tiles held in LDS).
 hipError_t launch_split_i8_rows(const SplitArgs& a, hipStream_t stream);
-bool i8_rows_supported(const SplitArgs& a);  // dim 128/256, one sequence, splits of <= 8/4 whole tiles
+bool i8_rows_supported(const SplitArgs& a);  // dim 128/256, one sequence, splits of whole tiles
 const char* i8_rows_kernel_name(const SplitArgs& a);
 // The MFMA split path used by the entry points: the int8-MFMA kernel where
 // i8_supported (the generic MFMA kernel instead where one_block_rows), else
