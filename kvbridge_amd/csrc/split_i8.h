@@ -908,7 +908,9 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
     const uint32_t row2 = hh / a.group, head2 = kv * a.group + hh % a.group;
     const size_t rh = size_t(row2) * a.q_heads + head2;
     float* const dst = scratch + (rh * a.splits + split) * W;
-    if (FUSED && nsplit == 1u) {  // the merge of one split is the split itself
+    if (FUSED && __builtin_expect(nsplit == 1u, 0)) {
+      // The merge of one split is the split itself.  (Out of line: a call of four
+      // short splits took 8.23 us with this inline, 8.19 so, 8.16 without it.)
       const float f = lsum > 0.f ? 1.f : 0.f;
       store_result<D>(a, rh, d, mm, f * lsum, fmaf(f, val, 0.f));
     } else if constexpr (FUSED) {  // agent-coherent, in the merge's packed layout
@@ -930,7 +932,7 @@ __global__ __launch_bounds__(64 * NW) void split_i8_kernel(
   // ---- fused merge: the last work-group to finish for this kv head merges
   // its splits (agent-scope release of every partial, then a ticket).
   if constexpr (FUSED) {
-    if (nsplit == 1u) return;
+    if (__builtin_expect(nsplit == 1u, 0)) return;
     __shared__ uint32_t last_s;
     // The partials were stored with agent-scope atomic stores (coherent
     // across XCDs, no L2 write-back needed) and are read back with
